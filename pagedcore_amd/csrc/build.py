@@ -55,6 +55,7 @@ FLAGS = [
 GUARDED_KERNELS: Dict[str, int] = {
     "paged_decode_bin_kernel": 2,
     "prefill_attention_kernel": 6,
+    "gemm_stream_kernel": 1,
 }
 
 _NOISE = "packed-fp32-ops' is not a recognized feature"

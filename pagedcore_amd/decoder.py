@@ -246,7 +246,11 @@ def _check_weights(weights: TinyLlamaWeights, what: str) -> None:
 # Shapes the kernel does not take (more rows, K not a multiple of 64, ...) use F.linear.
 # Split counts measured on the batch-128 step: q|k|v at 2 (160 workgroups of 32-row tiles,
 # half the partials of 4) 1.930 vs 1.950 ms; o_proj at 2 or 8 and down at 4 or 16 no better.
+# Up to 64 rows half as many for o_proj and down: the kernel that runs there fills the GPU
+# with them (o_proj 3.4-4.1 us at 2 splits, 3.4-4.4 at 4; down 5.9-8.5 at 4, 6.0-7.8 at 8) and
+# the norm that sums the partials reads half.
 GEMM_M128_ROWS = 128
+GEMM_FEW_ROWS = 64
 QKV_SPLITS = 2
 O_PROJ_SPLITS = 4
 DOWN_SPLITS = 8
@@ -298,10 +302,11 @@ def _attention_block(
     the caller; qkv fp16 [rows, 2560] or fp32 partial sums [splits, rows, 2560]), o_proj +
     residual + RMSNorm, SwiGLU MLP + residual + the next RMSNorm (reference
     src/pagedcore/decoder.py:173-193)."""
+    fewer = 2 if x.shape[0] <= GEMM_FEW_ROWS else 1
     attention = attend(_linear_parts(x, fused.qkv, QKV_SPLITS))
-    _add_rms_norm(x, hidden, _linear_parts(attention, layer.o_proj, O_PROJ_SPLITS), layer.post_attention_norm)
+    _add_rms_norm(x, hidden, _linear_parts(attention, layer.o_proj, O_PROJ_SPLITS // fewer), layer.post_attention_norm)
     activated = _swiglu(x, fused.gate_up)
-    _add_rms_norm(x, hidden, _linear_parts(activated, layer.down_proj, DOWN_SPLITS), following_norm)
+    _add_rms_norm(x, hidden, _linear_parts(activated, layer.down_proj, DOWN_SPLITS // fewer), following_norm)
 
 
 def _check_gpu(allocator: KVAllocator, weights: TinyLlamaWeights, what: str) -> None:

@@ -201,3 +201,40 @@ def test_gemm_swiglu_permutes_exactly(device):
     assert torch.equal(run(x[rows], w), base[rows])
     permuted = torch.cat((w[:half][cols], w[half:][cols]))
     assert torch.equal(run(x, permuted), base[:, cols])
+
+
+# --- the streaming form: edges of its row tiles, column tiles and K units --------------------
+
+# (n, k, splits): one unit and one tile; odd units per wave, a last 24-column SwiGLU tile that
+# is partly outside (160 / 24), tiles not a multiple of 8; the decode step's shapes.
+STREAM_SHAPES = [(64, 64, 1), (320, 704, 1), (96, 1408, 2), (2560, 2048, 2), (2048, 5632, 4), (2048, 2048, 4)]
+
+
+@pytest.mark.parametrize("m", [1, 15, 16, 17, 32, 33, 48, 49, 64, 65, 97, 128])
+@pytest.mark.parametrize("n,k,splits", STREAM_SHAPES)
+def test_gemm_row_and_tile_edges(device, m, n, k, splits):
+    """Every row count at the edges of the row tiles: partials against fp32 split by split,
+    nothing written past the output, and with one split the fp16 and SwiGLU epilogues bit
+    equal to the rounded partials (the same sums under every epilogue)."""
+    x, w = _inputs(device, m, n, k, seed=3 * m + n + k)
+    guard = torch.full((splits * m * n + 64,), -77.0, dtype=torch.float32, device=device)
+    out = guard[: splits * m * n].view(splits, m, n).fill_(float("nan"))
+    _hip.gemm_m128(out, x, w, splits=splits, epilogue=_hip.GEMM_PARTIALS)
+    torch.cuda.synchronize()
+    assert (guard[splits * m * n :] == -77.0).all()
+    span = k // splits
+    for s in range(splits):
+        part = x[:, s * span : (s + 1) * span].float() @ w[:, s * span : (s + 1) * span].float().t()
+        scale = part.abs().max().item()
+        # fp32 accumulation of the same products in another order
+        assert (out[s] - part).abs().max().item() <= 2e-6 * scale + 1e-7
+    if splits == 1:
+        half = torch.empty((m, n), dtype=torch.float16, device=device)
+        _hip.gemm_m128(half, x, w, epilogue=_hip.GEMM_HALF)
+        fused = torch.empty((m, n // 2), dtype=torch.float16, device=device)
+        _hip.gemm_m128(fused, x, w, epilogue=_hip.GEMM_SWIGLU)
+        separate = torch.empty_like(fused)
+        _hip.silu_mul(separate, half)
+        torch.cuda.synchronize()
+        assert np.array_equal(_bits(half), _bits(out[0].half()))
+        assert np.array_equal(_bits(fused), _bits(separate))
