@@ -293,6 +293,16 @@ int pc_gemm_m128(void* out, const void* x, const void* w, int32_t m, int32_t n, 
                  int32_t epilogue, void* stream);
 
 /*
+ * The same product and epilogues for the rows of a prompt: m in [1, 65536], k up to 2^22, m * k,
+ * n * k and splits * m * n up to 2^31, otherwise the shape and alignment rules of pc_gemm_m128.
+ *
+ * Replaces torch.nn.functional.linear on a prompt's activations (reference
+ * src/pagedcore/dense.py:91-104, called per layer by src/pagedcore/decoder.py:113-135).
+ */
+int pc_gemm_rows(void* out, const void* x, const void* w, int32_t m, int32_t n, int32_t k, int32_t splits,
+                 int32_t epilogue, void* stream);
+
+/*
  * Causal attention of one prompt over its contiguous K/V (the prefill of one sequence).
  *
  * Replaces the prompt's dense_attention (reference src/pagedcore/dense.py:69-81, called by

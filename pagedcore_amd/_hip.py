@@ -117,6 +117,8 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.pc_add_rms_norm_parts.argtypes = [_p, _p, _p, _i32, _p, _i64, _i32, ctypes.c_float, _p]
     lib.pc_gemm_m128.restype = ctypes.c_int
     lib.pc_gemm_m128.argtypes = [_p, _p, _p, _i32, _i32, _i32, _i32, _i32, _p]
+    lib.pc_gemm_rows.restype = ctypes.c_int
+    lib.pc_gemm_rows.argtypes = [_p, _p, _p, _i32, _i32, _i32, _i32, _i32, _p]
 
 
 def load() -> ctypes.CDLL:
@@ -464,6 +466,15 @@ def gemm_m128(out: Tensor, x: Tensor, w: Tensor, *, splits: int = 1, epilogue: i
     """Decode-step projection x @ w.T for up to 128 rows of x (pc_gemm_m128): x fp16 [m, k],
     w fp16 [n, k], both contiguous. out: fp32 [splits, m, n] (GEMM_PARTIALS), fp16 [m, n]
     (GEMM_HALF) or fp16 [m, n // 2] (GEMM_SWIGLU, w the stacked [gate | up] weight)."""
+    _gemm("pc_gemm_m128", out, x, w, splits, epilogue)
+
+
+def gemm_rows(out: Tensor, x: Tensor, w: Tensor, *, splits: int = 1, epilogue: int = GEMM_PARTIALS) -> None:
+    """gemm_m128 for the rows of a prompt (pc_gemm_rows): the same arguments, up to 65536 rows."""
+    _gemm("pc_gemm_rows", out, x, w, splits, epilogue)
+
+
+def _gemm(name: str, out: Tensor, x: Tensor, w: Tensor, splits: int, epilogue: int) -> None:
     lib = load()
     m, k = x.shape
     n = w.shape[0]
@@ -480,8 +491,10 @@ def gemm_m128(out: Tensor, x: Tensor, w: Tensor, *, splits: int = 1, epilogue: i
         raise HipExtensionError(f"out must be {expected[1]} {list(expected[0])}")
     if not (x.is_contiguous() and w.is_contiguous() and out.is_contiguous()):
         raise HipExtensionError("x, w and out must be contiguous")
-    status = lib.pc_gemm_m128(out.data_ptr(), x.data_ptr(), w.data_ptr(), m, n, k, splits, epilogue, _stream(x.device))
-    _check(lib, "pc_gemm_m128", status)
+    status = getattr(lib, name)(
+        out.data_ptr(), x.data_ptr(), w.data_ptr(), m, n, k, splits, epilogue, _stream(x.device)
+    )
+    _check(lib, name, status)
 
 
 def add_rms_norm(out: Tensor, hidden: Tensor, delta: Optional[Tensor], weight: Tensor, eps: float = 1e-5) -> None:

@@ -21,7 +21,7 @@ from typing import Dict, Iterable, List, Mapping
 HERE = os.path.dirname(os.path.abspath(__file__))
 PACKAGE = os.path.dirname(HERE)
 ROOT = os.path.dirname(PACKAGE)
-SOURCES = [os.path.join(HERE, name) for name in ("pagedcore_hip.hip", "decode_step.hip", "prefill.hip", "skinny_gemm.hip")]
+SOURCES = [os.path.join(HERE, name) for name in ("pagedcore_hip.hip", "decode_step.hip", "prefill.hip", "skinny_gemm.hip", "tile_gemm.hip")]
 OUTPUT = os.path.join(PACKAGE, "libpagedcore_hip.so")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 
@@ -56,6 +56,7 @@ GUARDED_KERNELS: Dict[str, int] = {
     "paged_decode_bin_kernel": 2,
     "prefill_attention_kernel": 6,
     "gemm_stream_kernel": 1,
+    "gemm_tile_kernel": 1,
 }
 
 _NOISE = "packed-fp32-ops' is not a recognized feature"

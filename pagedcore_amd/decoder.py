@@ -20,8 +20,9 @@ decode step is one batch-wide pass per layer:
   logits = x @ Wlm^T                                          GEMM (hipBLASLt via torch)
 
 The projections run on pc_gemm_m128 at up to 128 rows (the split-K partial sums are added
-and rounded to fp16 once by the kernel that consumes them) and on F.linear (hipBLASLt)
-otherwise, with pc_silu_mul for the SwiGLU. Every elementwise kernel rounds to fp16 where
+and rounded to fp16 once by the kernel that consumes them); above that, a prompt's rows among
+them, on pc_gemm_rows or on F.linear (hipBLASLt), whichever is faster at the shape (_rows_splits,
+_rows_swiglu), with pc_silu_mul for the SwiGLU after F.linear. Every elementwise kernel rounds to fp16 where
 the reference's torch expression does (see the kernels' comments), so a row's result
 differs from the reference only by fp32 summation order inside the GEMMs, the norms and the
 attention.
@@ -240,10 +241,12 @@ def _check_weights(weights: TinyLlamaWeights, what: str) -> None:
         raise ValueError(f"paged {what} requires 22 decoder layers")
 
 
-# Decode steps of up to GEMM_M128_ROWS rows run their q|k|v, o_proj, gate|up and down
-# projections on pc_gemm_m128: q|k|v, o_proj and down as fp32 split-K partial sums (summed
-# and rounded once by the RoPE / residual-add consumers), gate|up with the SwiGLU epilogue.
-# Shapes the kernel does not take (more rows, K not a multiple of 64, ...) use F.linear.
+# Up to GEMM_M128_ROWS rows (a decode step, a short prompt) the q|k|v, o_proj, gate|up and down
+# projections run on pc_gemm_m128: q|k|v, o_proj and down as fp32 split-K partial sums (summed
+# and rounded once by the RoPE / residual-add consumers), gate|up with the SwiGLU epilogue; a
+# 128-token prompt's four take 40 us there, 58 with hipBLASLt and pc_silu_mul. More rows go to
+# pc_gemm_rows where that is faster. Operands the kernels do not take (K not a multiple of
+# 64, strided or misaligned weights, ...) use F.linear.
 # Split counts measured on the batch-128 step: q|k|v at 2 (160 workgroups of 32-row tiles,
 # half the partials of 4) 1.930 vs 1.950 ms; o_proj at 2 or 8 and down at 4 or 16 no better.
 # Up to 64 rows half as many for o_proj and down: the kernel that runs there fills the GPU
@@ -256,13 +259,68 @@ O_PROJ_SPLITS = 4
 DOWN_SPLITS = 8
 
 
-def _linear_parts(x: Tensor, weight: Tensor, preferred_splits: int) -> Tensor:
-    """x @ weight.T: fp32 split-K partial sums [splits, rows, n] from pc_gemm_m128 (the most
-    splits up to preferred_splits whose K ranges are multiples of 64), or the fp16 product
-    [rows, n] of F.linear when the shape does not fit that kernel."""
+def _rows_splits(rows: int, n: int, k: int) -> int:
+    """K splits for pc_gemm_rows above GEMM_M128_ROWS rows, or 0 where F.linear (hipBLASLt) is
+    the faster product. By the count of 128 x 128 tiles against the 256 CUs: few tiles want K
+    split (a long K more), and pay for it in partials that the consumer reads; about one per
+    two CUs still win unsplit; more are the library's. Measured, us here / library (the
+    consumer reads the partials in 1-3 us): o_proj 7.1 / 9.4 at 256 rows and 9.2 / 11.2 at 512
+    (2 splits), 13.8 / 15.6 at 1024 (unsplit), 22.1 / 22.1 at 2048; q|k|v 9.2 / 10.7 at 384 (2),
+    13.6 / 15.0 at 768 (unsplit), 12.8 / 13.2 at 512, 28.0 / 27.8 at 2048; down 14.5 / 20.6 at
+    256, 19.1 / 28.0 at 512, 24.2 / 32.8 at 640 (4), 31.3 / 40.0 at 1024 (2), 30.0 / 32.4 at 768
+    (2), 56.8 / 55.8 at 2048."""
+    tiles = -(-rows // 128) * -(-n // 128)
+    if k >= 4096:
+        return 4 if tiles <= 80 else 2 if 100 < tiles <= 128 else 0
+    return 2 if tiles <= 64 else 1 if 100 <= tiles <= 128 else 0
+
+
+def _rows_swiglu(rows: int, width: int) -> bool:
+    """Whether pc_gemm_rows runs the SwiGLU projection faster than F.linear + pc_silu_mul: up to
+    one workgroup per CU of 128 x 128 tiles (outputs), or two per CU of 128 x 96, always; beyond
+    that when the last round of 128 x 96 tiles is not mostly empty (1536 rows 77.6 / 84.7 us,
+    2048 rows 95.6 / 101.7; 1280 rows, 590 tiles on 1024 places, 70.6 / 60.1)."""
+    row_tiles = -(-rows // 128)
+    if row_tiles * -(-width // 128) <= 256:
+        return True
+    tiles = row_tiles * -(-width // 96)
+    return tiles <= 512 or 3 * tiles >= 2 * 512 * -(-tiles // 512)
+
+
+def _kernel_operands(x: Tensor, weight: Tensor) -> bool:
+    """Contiguous fp16 operands on 16-byte boundaries, as the GEMM kernels read them."""
+    return all(
+        t.dtype == torch.float16 and t.is_contiguous() and t.data_ptr() % 16 == 0 for t in (x, weight)
+    )
+
+
+def _linear_rows(x: Tensor, weight: Tensor) -> Tensor:
+    """x @ weight.T above GEMM_M128_ROWS rows: fp32 partial sums or the fp16 product of
+    pc_gemm_rows, or F.linear where that is faster or the shape does not fit the kernel."""
     rows, k = x.shape
     n = weight.shape[0]
-    if rows <= GEMM_M128_ROWS and n % 32 == 0 and x.is_contiguous() and weight.is_contiguous():
+    splits = _rows_splits(rows, n, k)
+    if splits and n % 32 == 0 and k % (64 * splits) == 0 and _kernel_operands(x, weight):
+        if splits > 1:
+            parts = torch.empty((splits, rows, n), dtype=torch.float32, device=x.device)
+            _hip.gemm_rows(parts, x, weight, splits=splits)
+            return parts
+        product = torch.empty((rows, n), dtype=torch.float16, device=x.device)
+        _hip.gemm_rows(product, x, weight, epilogue=_hip.GEMM_HALF)
+        return product
+    return F.linear(x, weight)
+
+
+def _linear_parts(x: Tensor, weight: Tensor, preferred_splits: int) -> Tensor:
+    """x @ weight.T: fp32 split-K partial sums [splits, rows, n] from pc_gemm_m128 (the most
+    splits up to preferred_splits whose K ranges are multiples of 64), _linear_rows above
+    GEMM_M128_ROWS rows, or the fp16 product [rows, n] of F.linear when the shape does not
+    fit the kernel."""
+    rows, k = x.shape
+    n = weight.shape[0]
+    if rows > GEMM_M128_ROWS:
+        return _linear_rows(x, weight)
+    if n % 32 == 0 and _kernel_operands(x, weight):
         splits = preferred_splits
         while splits >= 1:
             if k % (64 * splits) == 0:
@@ -275,12 +333,15 @@ def _linear_parts(x: Tensor, weight: Tensor, preferred_splits: int) -> Tensor:
 
 def _swiglu(x: Tensor, gate_up: Tensor) -> Tensor:
     """fp16(fp16(silu(x @ gate.T)) * fp16(x @ up.T)) for the stacked [gate | up] weight:
-    one pc_gemm_m128 launch with the SwiGLU epilogue, or F.linear + pc_silu_mul."""
+    one GEMM launch with the SwiGLU epilogue, or F.linear + pc_silu_mul."""
     rows, k = x.shape
     n = gate_up.shape[0]
     activated = torch.empty((rows, n // 2), dtype=torch.float16, device=x.device)
-    if rows <= GEMM_M128_ROWS and n % 64 == 0 and k % 64 == 0 and x.is_contiguous() and gate_up.is_contiguous():
+    fits = n % 64 == 0 and k % 64 == 0 and _kernel_operands(x, gate_up)
+    if fits and rows <= GEMM_M128_ROWS:
         _hip.gemm_m128(activated, x, gate_up, epilogue=_hip.GEMM_SWIGLU)
+    elif fits and _rows_swiglu(rows, n // 2):
+        _hip.gemm_rows(activated, x, gate_up, epilogue=_hip.GEMM_SWIGLU)
     else:
         _hip.silu_mul(activated, F.linear(x, gate_up))
     return activated
@@ -668,21 +729,17 @@ def _prefill_forward(ids: Tensor, positions: Tensor, slots: Tensor, weights: Tin
     query = torch.empty((tokens, Q_HEADS, HEAD_DIM), dtype=torch.float16, device=device)
     attended = torch.empty_like(query)
     for index, layer in enumerate(weights.layers):
-        fused = _fused(layer)
-        qkv = F.linear(x, fused.qkv)
-        _hip.rope_kv_append(query, qkv, positions, table, key_out=key, value_out=value, pool=pool, layer=index,
-                            slot_mapping=slots)
-        if on_layer is not None:
-            on_layer(index)
-        _hip.prefill_attention(attended, query, key, value)
-        projected = F.linear(attended.view(tokens, HIDDEN), layer.o_proj)
-        _hip.add_rms_norm(x, hidden, projected, layer.post_attention_norm, RMS_EPS)
-        gate_up = F.linear(x, fused.gate_up)
-        activated = torch.empty((tokens, gate_up.shape[1] // 2), dtype=torch.float16, device=device)
-        _hip.silu_mul(activated, gate_up)
-        down = F.linear(activated, layer.down_proj)
+
+        def attend(qkv: Tensor, index: int = index) -> Tensor:
+            rope = _hip.rope_kv_append_parts if qkv.ndim == 3 else _hip.rope_kv_append
+            rope(query, qkv, positions, table, key_out=key, value_out=value, pool=pool, layer=index, slot_mapping=slots)
+            if on_layer is not None:
+                on_layer(index)
+            _hip.prefill_attention(attended, query, key, value)
+            return attended.view(tokens, HIDDEN)
+
         following = weights.layers[index + 1].input_norm if index + 1 < LAYERS else weights.final_norm
-        _hip.add_rms_norm(x, hidden, down, following, RMS_EPS)
+        _attention_block(x, hidden, layer, _fused(layer), following, attend)
     return x
 
 

@@ -8,6 +8,7 @@ import pytest
 import torch
 
 from oracle import decoder_reference as dref
+from pagedcore_amd import _hip
 from pagedcore_amd import decoder as dec
 from pagedcore_amd.engine_types import KVReservation, RequestId
 from pagedcore_amd.kv_cache import KVAllocator
@@ -128,3 +129,70 @@ def test_fused_decode_write_checks_before_any_write():
         assert positions.tolist() == [5, 16]
         assert slots.tolist() == [allocator.block_table(requests[0])[0] * 16 + 5, allocator._decode_appends[requests[1]].sequence.blocks[1] * 16]
     assert allocator.capacity() == counts
+
+
+@pytest.mark.parametrize("rows", [1, 64, 128, 129, 384, 640, 1024, 2048])
+@pytest.mark.parametrize("form", ["plain", "strided", "misaligned", "odd_k", "odd_n"])
+def test_projection_route_takes_only_what_the_kernels_read(monkeypatch, rows, form):
+    """_linear_parts and _swiglu hand the GEMM kernels contiguous, aligned operands whose K
+    divides into 64-column splits, and give every other form to the library product, bit for
+    bit. The kernels are stood in for by fp32 products of the same arguments."""
+    n, k = (96 if form == "odd_n" else 128), (72 if form == "odd_k" else 256)
+    n += 1 if form == "odd_n" else 0
+    gen = torch.Generator().manual_seed(rows)
+    x = torch.randn((rows, k), generator=gen).half()
+    if form == "strided":
+        weight = torch.randn((n, 2 * k), generator=gen).half()[:, ::2]
+    elif form == "misaligned":
+        weight = torch.randn(n * k + 1, generator=gen).half()[1:].view(n, k)
+    else:
+        weight = torch.randn((n, k), generator=gen).half()
+    calls = []
+
+    def stand_in(out, x, w, *, splits=1, epilogue=_hip.GEMM_PARTIALS):
+        calls.append(epilogue)
+        assert x.is_contiguous() and w.is_contiguous() and w.data_ptr() % 16 == 0
+        assert w.shape[0] % 32 == 0 and w.shape[1] % (64 * splits) == 0
+        if epilogue == _hip.GEMM_SWIGLU:
+            assert w.shape[0] % 64 == 0
+            y = (x.float() @ w.float().t()).half().float()
+            half = w.shape[0] // 2
+            out.copy_((torch.nn.functional.silu(y[:, :half]).half().float() * y[:, half:]).half())
+            return
+        span = w.shape[1] // splits
+        products = [x[:, s * span : (s + 1) * span].float() @ w[:, s * span : (s + 1) * span].float().t() for s in range(splits)]
+        out.copy_(torch.stack(products) if epilogue == _hip.GEMM_PARTIALS else products[0].half())
+
+    def silu_mul(out, gate_up):
+        half = gate_up.shape[1] // 2
+        out.copy_((torch.nn.functional.silu(gate_up[:, :half].float()).half().float() * gate_up[:, half:].float()).half())
+
+    monkeypatch.setattr(_hip, "gemm_m128", stand_in)
+    monkeypatch.setattr(_hip, "gemm_rows", stand_in)
+    monkeypatch.setattr(_hip, "silu_mul", silu_mul)
+    library = torch.nn.functional.linear(x, weight)
+    got = dec._linear_parts(x, weight, 4)
+    got = got.sum(0).half() if got.ndim == 3 else got
+    if form == "plain":
+        assert calls == [_hip.GEMM_PARTIALS]
+        # one fp16 rounding of sums taken in another order
+        torch.testing.assert_close(got, library, atol=2e-3 * library.abs().max().item(), rtol=0)
+    else:
+        assert calls == [] and torch.equal(got, library)
+    if form != "odd_n":
+        calls.clear()
+        fused = dec._swiglu(x, weight)
+        expected = torch.empty_like(fused)
+        silu_mul(expected, library)
+        assert calls == ([_hip.GEMM_SWIGLU] if form == "plain" else [])
+        torch.testing.assert_close(fused, expected, atol=4e-3 * expected.abs().max().item(), rtol=0)
+
+
+@pytest.mark.parametrize("n,k", [(2560, 2048), (2048, 2048), (2048, 5632), (32000, 2048), (128, 64)])
+def test_rows_splits_always_divide_into_the_decoders_shapes(n, k):
+    for rows in range(129, 2049):
+        splits = dec._rows_splits(rows, n, k)
+        assert splits in (0, 1, 2, 4)
+        if splits > 1:
+            # the partials stay a fraction of the weight they save reading late
+            assert splits * rows * n * 4 <= 32 << 20

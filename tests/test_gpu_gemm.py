@@ -238,3 +238,51 @@ def test_gemm_row_and_tile_edges(device, m, n, k, splits):
         torch.cuda.synchronize()
         assert np.array_equal(_bits(half), _bits(out[0].half()))
         assert np.array_equal(_bits(fused), _bits(separate))
+
+
+# --- pc_gemm_rows (a prompt's rows) -----------------------------------------------------------
+
+# (n, k, splits, rows): every tile shape of the dispatch (64 x 64, 64 x 128, 128 x 128,
+# 128 x 192; SwiGLU 64, 96 and 128 output columns, and 96 on two stages), rows one short of, at
+# and one past a tile, column counts that end inside a tile, fewer K stages than the ring has.
+ROWS_SHAPES = [
+    (64, 64, 1, (1, 63, 64, 65, 200)),
+    (352, 128, 1, (129, 255)),
+    (2560, 2048, 2, (129, 192, 256, 333)),
+    (2048, 5632, 4, (129, 300, 513)),
+    (2080, 1408, 2, (641, 1025)),
+    (11264, 256, 1, (129, 300, 600, 700)),
+]
+
+
+@pytest.mark.parametrize("n,k,splits,m", [(n, k, s, m) for n, k, s, rows in ROWS_SHAPES for m in rows])
+def test_gemm_rows_tiles(device, m, n, k, splits):
+    """Partials against fp32 split by split, nothing written past the output; with one split the
+    fp16 epilogue bit equal to the rounded partials, and SwiGLU within the rounding of its
+    two projections of pc_silu_mul of them (its tiles may differ, the K order does not)."""
+    x, w = _inputs(device, m, n, k, seed=5 * m + n + k)
+    guard = torch.full((splits * m * n + 64,), -77.0, dtype=torch.float32, device=device)
+    out = guard[: splits * m * n].view(splits, m, n).fill_(float("nan"))
+    _hip.gemm_rows(out, x, w, splits=splits, epilogue=_hip.GEMM_PARTIALS)
+    torch.cuda.synchronize()
+    assert (guard[splits * m * n :] == -77.0).all()
+    span = k // splits
+    for s in range(splits):
+        xs, ws = x[:, s * span : (s + 1) * span].double(), w[:, s * span : (s + 1) * span].double()
+        # `span` exact products added in fp32, whatever the order: each of at most `span`
+        # additions rounds by 2^-24 of a partial sum no larger than the sum of magnitudes.
+        bound = span * 2.0**-24 * (xs.abs() @ ws.abs().t())
+        assert ((out[s].double() - xs @ ws.t()).abs() <= bound).all()
+    if splits == 1:
+        half = torch.empty((m, n), dtype=torch.float16, device=device)
+        _hip.gemm_rows(half, x, w, epilogue=_hip.GEMM_HALF)
+        torch.cuda.synchronize()
+        assert np.array_equal(_bits(half), _bits(out[0].half()))
+        if n % 64 == 0:
+            fused = torch.full((m * (n // 2) + 64,), -77.0, dtype=torch.float16, device=device)
+            _hip.gemm_rows(fused[: m * (n // 2)].view(m, n // 2), x, w, epilogue=_hip.GEMM_SWIGLU)
+            separate = torch.empty((m, n // 2), dtype=torch.float16, device=device)
+            _hip.silu_mul(separate, half)
+            torch.cuda.synchronize()
+            assert (fused[m * (n // 2) :] == -77.0).all()
+            assert np.array_equal(_bits(fused[: m * (n // 2)]), _bits(separate.view(-1)))
