@@ -54,7 +54,7 @@ FLAGS = [
 # the kernel's launch shape relies on. Each must report no scratch and no spills.
 GUARDED_KERNELS: Dict[str, int] = {
     "paged_decode_bin_kernel": 2,
-    "prefill_attention_kernel": 6,
+    "prefill_attention_kernel": 4,
     "gemm_stream_kernel": 1,
     "gemm_tile_kernel": 1,
 }

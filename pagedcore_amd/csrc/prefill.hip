@@ -4,20 +4,31 @@
 // with q [T][32][64], k and v [T][4][64] (the rotated keys and the values that
 // pc_rope_kv_append wrote), o [T][32][64], all fp16.
 //
-// Work split: one workgroup per (16-query block, kv head), longest (latest) blocks first; its
-// 8 waves are the 8 query heads of the kv head. Each 16-key block of K and V is staged in
-// LDS once per workgroup (LDS DMA by four of the waves, two buffers, one barrier per block)
-// and read by all eight waves. A wave walks key blocks 0 .. its query block with an online
-// softmax in fp32:
+// Work split: one workgroup per (16-query block, four query heads), one wave per head; two
+// workgroups share a kv head. The workgroup stages 64 keys of K and V at a time in LDS (LDS
+// DMA, two stages, one barrier per step) and every wave reads them. With KG = 2 a second set of
+// four waves takes every other step, and the two sets' results meet in LDS at the end. A wave
+// walks key blocks 0 .. its query block with an online softmax in fp32:
 //   S^T = K_blk . Q^T   on v_mfma_f32_16x16x32_f16 (lane (c, g): keys 4g..4g+3 of position c)
-//   O^T += V^T . P^T    on v_mfma_f32_16x16x16f16, V^T from the decode kernel's transposing
-//                       LDS reads, P^T straight from the S^T registers
-//   l   += 1 . P^T      one more v_mfma_f32_16x16x16f16 with an all-ones A operand: the
-//                       softmax denominator of every position, summed on the matrix core
+//   O^T += V^T . P^T    on v_mfma_f32_16x16x32_f16 over pairs of blocks, V^T from the decode
+//                       kernel's transposing LDS reads, P^T straight from the S^T registers
+//   l   += 1 . P^T      one more MFMA with an all-ones A operand: the softmax denominator of
+//                       every position, summed on the matrix core
 // so every per-position quantity (running max, sum, rescale) stays in the lane that owns
 // the position. Only the diagonal block needs the causal mask. Probabilities enter the PV
 // product as fp16 (relative error 2^-11) and the denominator sums those same fp16 weights;
 // everything else is fp32 with one final fp16 rounding.
+//
+// What bounds it: a step of 64 keys is a chain (barrier, K from LDS, MFMA, max, exp, MFMA) of
+// about 1400 cycles for a wave alone on its SIMD, 440 of them VALU issue and 290 matrix work.
+// Short prompts run that chain with the chip half empty, so they get the two key sets (half
+// the chain) and small workgroups; long ones need every SIMD kept full to the end, so heavy and
+// light query blocks are paired on a CU (kSnake). All K fragments of a step, and all V fragments,
+// are read in one block each: two exposed LDS latencies per step instead of six. Measured, us
+// per layer, against eight waves per workgroup without these (same outputs bit for bit for
+// KG = 1): 64 tokens 3.8 -> 3.1, 333 7.3 -> 5.7, 512 9.0 -> 6.9, 1024 14.8 -> 10.6, 2048 31.1 ->
+// 26.5. Slower: three stages (28.7 at 2048, 6.7 at 333), 32 queries per wave (34.2), packed
+// fp16 conversion (29.8 against 28.6), K prefetched across steps.
 
 #include <hip/hip_runtime.h>
 
@@ -42,14 +53,17 @@ using pc_internal::set_error;
 constexpr int kKVHeads = 4;
 constexpr int kQHeads = 32;
 constexpr int kHeadDim = 64;
-constexpr int kWaves = kQHeads / kKVHeads;  // 8 query heads per workgroup
-constexpr int kThreads = 64 * kWaves;
+constexpr int kHeads = 4;                    // query heads (waves of a key set) per workgroup
+constexpr int kPerKV = kQHeads / kKVHeads / kHeads;  // workgroups per kv head and query block
+constexpr int kPerBlock = kKVHeads * kPerKV;         // workgroups per query block
+constexpr int kSnake = 256;                  // one workgroup per CU
 constexpr int kBlock = 16;                   // positions per query block and keys per key block
 constexpr int kTileBytes = kBlock * kHeadDim * 2;  // 16 rows of one kv head: 2 KiB
 constexpr int kBufBytes = 2 * kTileBytes;           // one key block: K tile, then V tile
-constexpr int kStepBlocks = 4;                      // key blocks per step (a multiple of 2)
+constexpr int kStepBlocks = 4;                      // key blocks per step
 constexpr int kStageBytes = kStepBlocks * kBufBytes;
 constexpr int kMaxTokens = 1 << 16;
+constexpr float kFloatMax = 3.402823466e38f;
 constexpr float kLazyLog2 = 8.0f;            // headroom (log2 of p) before the running max is raised
 
 // f(integral_constant<int, p>) for every pair p of key blocks of a step, in order.
@@ -76,22 +90,36 @@ struct PrefillArgs {
   _Float16* out;
 };
 
-// Scalar parameters in the order of PrefillArgs: all are preloaded into SGPRs at wave
-// launch.
-__global__ __launch_bounds__(kThreads) void prefill_attention_kernel(const _Float16* q, const _Float16* k,
-                                                                     const _Float16* v, int tokens, _Float16* out) {
+// KG key sets of kHeads waves each. Scalar parameters in the order of PrefillArgs: all are
+// preloaded into SGPRs at wave launch.
+template <int KG>
+__global__ __launch_bounds__(64 * kHeads * KG) void prefill_attention_kernel(const _Float16* q, const _Float16* k,
+                                                                             const _Float16* v, int tokens,
+                                                                             _Float16* out) {
   const PrefillArgs a{q, k, v, tokens, out};
-  // Two stages of kStepBlocks key blocks each: stage s, block b: K tile at s * kStageBytes +
-  // b * kBufBytes, its V tile kTileBytes after it.
-  __shared__ __attribute__((aligned(16))) char lds[2][kStageBytes];
-  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  // Per key set two stages of kStepBlocks key blocks each: stage s, block b: K tile at
+  // s * kStageBytes + b * kBufBytes, its V tile kTileBytes after it.
+  __shared__ __attribute__((aligned(16))) char smem[KG * 2 * kStageBytes];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int w = wave % kHeads, kg = wave / kHeads;
+  char* const lds = smem + kg * 2 * kStageBytes;
   const int lane = threadIdx.x & 63;
   const int c = lane & 15;
   const int g = lane >> 4;
   const int qblocks = (a.tokens + kBlock - 1) / kBlock;
-  const int h = blockIdx.x % kKVHeads;
-  const int qb = qblocks - 1 - static_cast<int>(blockIdx.x / kKVHeads);
-  const int head = kWaves * h + w;
+  // Latest (longest) query blocks first, in chunks of one workgroup per CU whose order turns
+  // round from chunk to chunk: the hardware deals a chunk to the CUs in turn, so a CU that got
+  // one of the longest of one chunk gets one of the shortest of the next (2048 tokens: a CU's
+  // blocks sum to 127 instead of 64 to 190; 31.1 -> 28.6 us).
+  int id = blockIdx.x;
+  const int chunk = id / kSnake, base = chunk * kSnake;
+  if (chunk & 1) {
+    const int in = id - base, blocks = min(kSnake, static_cast<int>(gridDim.x) - base) / kPerBlock;
+    id = base + (blocks - 1 - in / kPerBlock) * kPerBlock + in % kPerBlock;
+  }
+  const int h = id % kPerBlock / kPerKV;
+  const int qb = qblocks - 1 - id / kPerBlock;
+  const int head = kQHeads / kKVHeads * h + kHeads * (id % kPerKV) + w;
   const int pos = kBlock * qb + c;  // this lane's query position (column of S^T)
   const int last = a.tokens - 1;
 
@@ -99,20 +127,18 @@ __global__ __launch_bounds__(kThreads) void prefill_attention_kernel(const _Floa
   half8_t qa = *reinterpret_cast<const half8_t*>(qrow);
   half8_t qc = *reinterpret_cast<const half8_t*>(qrow + 32);
 
-  // Staging: every wave issues kStepBlocks / 2 LDS DMA instructions per stage (each 64 lanes
-  // x 16 B = rows srow .. srow + 7 of one tile): wave w stages blocks w / 4, w / 4 + 2, ...
-  // of the step, the K (w & 2 = 0) or V tile, rows 8 (w & 1) .. 8 (w & 1) + 7. K piece p of
-  // row r sits at position p ^ (r & 7) (the A-operand reads of 16 rows then hit 8 different
-  // 16 B bank groups); V uses the decode kernel's 32 B-group swizzle for its transposing
-  // reads.
+  // Staging: wave w of a key set issues kStepBlocks LDS DMA instructions per stage (each 64
+  // lanes x 16 B = rows srow .. srow + 7 of one tile): of every block, the K (w & 2 = 0) or V
+  // tile, rows 8 (w & 1) .. 8 (w & 1) + 7. K piece p of row r sits at position p ^ (r & 7) (the
+  // A-operand reads of 16 rows then hit 8 different 16 B bank groups); V uses the decode
+  // kernel's 32 B-group swizzle for its transposing reads.
   const bool stage_v = (w & 2) != 0;
-  const int sblock = w >> 2;
   const int qs = lane & 7;
   const int srow = 8 * (w & 1) + (lane >> 3);
   const int piece = stage_v ? 2 * ((qs >> 1) ^ row_sel(srow)) + (qs & 1) : qs ^ (srow & 7);
   const _Float16* ssrc = (stage_v ? a.v : a.k) + h * kHeadDim + 8 * piece;
-  const int sdst = sblock * kBufBytes + (stage_v ? kTileBytes : 0) + 1024 * (w & 1);
-  const uint32_t lds0 = lds_offset(lds[0]);
+  const int sdst = (stage_v ? kTileBytes : 0) + 1024 * (w & 1);
+  const uint32_t lds0 = lds_offset(lds);
   // K reads: lane (c, g) takes row c, pieces g and 4 + g
   const uint32_t kaddr0 = lds0 + c * 128 + 16 * (g ^ (c & 7));
   const uint32_t kaddr1 = lds0 + c * 128 + 16 * ((4 + g) ^ (c & 7));
@@ -120,15 +146,16 @@ __global__ __launch_bounds__(kThreads) void prefill_attention_kernel(const _Floa
   const int rr = 4 * g + (c >> 2);
   const uint32_t vbase = lds0 + kTileBytes + rr * 128 + 8 * (c & 3);
   const uint32_t tsel = row_sel(rr);
+  const uint32_t va[4] = {vbase + 32 * (0 ^ tsel), vbase + 32 * (1 ^ tsel), vbase + 32 * (2 ^ tsel), vbase + 32 * (3 ^ tsel)};
 
   // Key blocks kStepBlocks * j .. + kStepBlocks - 1 into stage `buf` (rows past the prompt
   // repeat its last row; their scores are masked).
   auto stage = [&](int j, int buf) {
 #pragma unroll
-    for (int i = 0; i < kStepBlocks / 2; ++i) {
-      const int row = min(kBlock * (kStepBlocks * j + sblock + 2 * i) + srow, last);
+    for (int b = 0; b < kStepBlocks; ++b) {
+      const int row = min(kBlock * (kStepBlocks * j + b) + srow, last);
       __builtin_amdgcn_global_load_lds(static_cast<const void*>(ssrc + static_cast<int64_t>(row) * kKVHeads * kHeadDim),
-                                       lds_ptr(lds[buf] + sdst + 2 * i * kBufBytes), 16, 0, 0);
+                                       lds_ptr(lds + buf * kStageBytes + sdst + b * kBufBytes), 16, 0, 0);
     }
     __builtin_amdgcn_sched_barrier(0);
   };
@@ -140,43 +167,50 @@ __global__ __launch_bounds__(kThreads) void prefill_attention_kernel(const _Floa
   for (int u = 0; u < 4; ++u) acc[u] = float4_t{0.f, 0.f, 0.f, 0.f};
   const int steps = (qb + kStepBlocks) / kStepBlocks;  // causal: key blocks 0 .. qb
 
-  // One step over the key blocks of step j, staged in stage B (a compile-time constant, so
+  const int rounds = (steps + KG - 1) / KG;
+
+  // Round J: each key set's step j = KG J + kg, staged in stage B (a compile-time constant, so
   // every LDS address below is a fixed base plus an immediate offset).
-  auto step = [&](int j, auto stage_index) {
+  auto step = [&](int J, auto stage_index) {
     constexpr int B = decltype(stage_index)::value;
     constexpr uint32_t so = B * kStageBytes;
+    const int j = KG * J + kg;
     // This wave's staging of step j (and, before the first step, Q) has landed; after the
     // barrier every wave's has, and every wave has finished reading the other stage (its
-    // reads of step j - 1 waited for lgkmcnt(0)), which the next staging refills. Q is named
-    // so that the compiler does not add a wait of its own for it, which would also wait for
-    // the staging issued below.
+    // reads of the round before waited for lgkmcnt(0)), which the next staging refills. Q is
+    // named so that the compiler does not add a wait of its own for it, which would also wait
+    // for the staging issued below.
     asm volatile("s_waitcnt vmcnt(0)" : "+v"(qa), "+v"(qc) : : "memory");
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_sched_barrier(0);
-    if (j + 1 < steps) stage(j + 1, B ^ 1);
+    if (j + KG < steps) stage(j + KG, B ^ 1);
+    if (KG > 1 && j >= steps) return;  // the last round of a set with no step left in it
     // sc[4 b + e]: key 4g + e of block kStepBlocks * j + b
     float sc[4 * kStepBlocks];
-    auto scores = [&](auto pair) {
-      constexpr int b = 2 * decltype(pair)::value;
-      half8_t k00, k01, k10, k11;
+    {
+      half8_t kf[8];
       asm volatile(
-          "ds_read_b128 %0, %4 offset:%6\n\tds_read_b128 %1, %5 offset:%6\n\tds_read_b128 %2, %4 offset:%7\n\t"
-          "ds_read_b128 %3, %5 offset:%7\n\ts_waitcnt lgkmcnt(0)"
-          : "=&v"(k00), "=&v"(k01), "=&v"(k10), "=&v"(k11)
-          : "v"(kaddr0), "v"(kaddr1), "i"(so + b * kBufBytes), "i"(so + (b + 1) * kBufBytes)
+          "ds_read_b128 %0, %8 offset:%10\n\tds_read_b128 %1, %9 offset:%10\n\t"
+          "ds_read_b128 %2, %8 offset:%11\n\tds_read_b128 %3, %9 offset:%11\n\t"
+          "ds_read_b128 %4, %8 offset:%12\n\tds_read_b128 %5, %9 offset:%12\n\t"
+          "ds_read_b128 %6, %8 offset:%13\n\tds_read_b128 %7, %9 offset:%13\n\t"
+          "s_waitcnt lgkmcnt(0)"
+          : "=&v"(kf[0]), "=&v"(kf[1]), "=&v"(kf[2]), "=&v"(kf[3]), "=&v"(kf[4]), "=&v"(kf[5]), "=&v"(kf[6]),
+            "=&v"(kf[7])
+          : "v"(kaddr0), "v"(kaddr1), "i"(so), "i"(so + kBufBytes), "i"(so + 2 * kBufBytes), "i"(so + 3 * kBufBytes)
           : "memory");
-      float4_t s0 = {0.f, 0.f, 0.f, 0.f}, s1 = {0.f, 0.f, 0.f, 0.f};
-      s0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(k00, qa, s0, 0, 0, 0);
-      s1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(k10, qa, s1, 0, 0, 0);
-      s0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(k01, qc, s0, 0, 0, 0);
-      s1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(k11, qc, s1, 0, 0, 0);
+      float4_t s[4];
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        sc[4 * b + e] = s0[e];
-        sc[4 * b + 4 + e] = s1[e];
+      for (int b = 0; b < 4; ++b) {
+        s[b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf[2 * b], qa, float4_t{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
       }
-    };
-    for_pairs(scores);
+#pragma unroll
+      for (int b = 0; b < 4; ++b) s[b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf[2 * b + 1], qc, s[b], 0, 0, 0);
+#pragma unroll
+      for (int b = 0; b < 4; ++b)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) sc[4 * b + e] = s[b][e];
+    }
     if (kStepBlocks * j + kStepBlocks - 1 >= qb) {  // the diagonal step: keys after the position, or past the prompt, are masked
 #pragma unroll
       for (int e = 0; e < 4 * kStepBlocks; ++e) {
@@ -187,8 +221,10 @@ __global__ __launch_bounds__(kThreads) void prefill_attention_kernel(const _Floa
     float bm = sc[0];
 #pragma unroll
     for (int e = 1; e < 4 * kStepBlocks; ++e) bm = fmaxf(bm, sc[e]);
-    if (j == 0) {
-      m = max_over_groups(bm);  // finite: key 0 is visible to every position
+    if (J == 0) {
+      // A step's first key is visible to every position; the bound keeps the max finite where
+      // infinite inputs make all 64 scores -inf (their weights are then 0, not NaN).
+      m = fmaxf(max_over_groups(bm), -kFloatMax);
       mc = m * kScoreToLog2;
     } else if (__builtin_amdgcn_ballot_w64(bm * kScoreToLog2 > mc + kLazyLog2) != 0) {
       const float mn = fmaxf(m, max_over_groups(bm));
@@ -199,6 +235,24 @@ __global__ __launch_bounds__(kThreads) void prefill_attention_kernel(const _Floa
       m = mn;
       mc = m * kScoreToLog2;
     }
+    __builtin_amdgcn_sched_barrier(0);
+    short4_t vt[16];  // vt[4 b + u]: block b, dims 16 u .. 16 u + 15
+    asm volatile(
+        "ds_read_b64_tr_b16 %0, %16 offset:%20\n\tds_read_b64_tr_b16 %1, %17 offset:%20\n\t"
+        "ds_read_b64_tr_b16 %2, %18 offset:%20\n\tds_read_b64_tr_b16 %3, %19 offset:%20\n\t"
+        "ds_read_b64_tr_b16 %4, %16 offset:%21\n\tds_read_b64_tr_b16 %5, %17 offset:%21\n\t"
+        "ds_read_b64_tr_b16 %6, %18 offset:%21\n\tds_read_b64_tr_b16 %7, %19 offset:%21\n\t"
+        "ds_read_b64_tr_b16 %8, %16 offset:%22\n\tds_read_b64_tr_b16 %9, %17 offset:%22\n\t"
+        "ds_read_b64_tr_b16 %10, %18 offset:%22\n\tds_read_b64_tr_b16 %11, %19 offset:%22\n\t"
+        "ds_read_b64_tr_b16 %12, %16 offset:%23\n\tds_read_b64_tr_b16 %13, %17 offset:%23\n\t"
+        "ds_read_b64_tr_b16 %14, %18 offset:%23\n\tds_read_b64_tr_b16 %15, %19 offset:%23\n\t"
+        "s_waitcnt lgkmcnt(0)"
+        : "=&v"(vt[0]), "=&v"(vt[1]), "=&v"(vt[2]), "=&v"(vt[3]), "=&v"(vt[4]), "=&v"(vt[5]), "=&v"(vt[6]),
+          "=&v"(vt[7]), "=&v"(vt[8]), "=&v"(vt[9]), "=&v"(vt[10]), "=&v"(vt[11]), "=&v"(vt[12]), "=&v"(vt[13]),
+          "=&v"(vt[14]), "=&v"(vt[15])
+        : "v"(va[0]), "v"(va[1]), "v"(va[2]), "v"(va[3]), "i"(so), "i"(so + kBufBytes), "i"(so + 2 * kBufBytes),
+          "i"(so + 3 * kBufBytes)
+        : "memory");
     // Per pair of blocks, P^T as one 32-key B operand: element e is key 4g + (e & 3) of
     // the pair's block e / 4; the V^T A operands concatenate the two blocks in the same
     // order.
@@ -207,22 +261,44 @@ __global__ __launch_bounds__(kThreads) void prefill_attention_kernel(const _Floa
       half8_t pb;
 #pragma unroll
       for (int e = 0; e < 8; ++e) pb[e] = static_cast<_Float16>(exp2_fast(fmaf(sc[4 * b + e], kScoreToLog2, -mc)));
-      short4_t a0, a1, a2, a3, b0, b1, b2, b3;
-      read_v_tiles<so + b * kBufBytes>(vbase, tsel, a0, a1, a2, a3);
-      read_v_tiles<so + (b + 1) * kBufBytes>(vbase, tsel, b0, b1, b2, b3);
-      acc[0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(join(a0, b0), pb, acc[0], 0, 0, 0);
-      acc[1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(join(a1, b1), pb, acc[1], 0, 0, 0);
-      acc[2] = __builtin_amdgcn_mfma_f32_16x16x32_f16(join(a2, b2), pb, acc[2], 0, 0, 0);
-      acc[3] = __builtin_amdgcn_mfma_f32_16x16x32_f16(join(a3, b3), pb, acc[3], 0, 0, 0);
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        acc[u] = __builtin_amdgcn_mfma_f32_16x16x32_f16(join(vt[4 * b + u], vt[4 * b + 4 + u]), pb, acc[u], 0, 0, 0);
       lacc = __builtin_amdgcn_mfma_f32_16x16x32_f16(ones, pb, lacc, 0, 0, 0);
     };
     for_pairs(accumulate);
   };
 
-  stage(0, 0);
-  for (int j = 0; j < steps; j += 2) {
-    step(j, std::integral_constant<int, 0>{});
-    if (j + 1 < steps) step(j + 1, std::integral_constant<int, 1>{});
+  if (kg < steps) stage(kg, 0);
+  for (int J = 0; J < rounds; J += 2) {
+    step(J, std::integral_constant<int, 0>{});
+    if (J + 1 < rounds) step(J + 1, std::integral_constant<int, 1>{});
+  }
+
+  if constexpr (KG == 2) {
+    // The second set leaves its accumulators, max and sum in LDS (over the stages, once every
+    // wave is done with them); the first folds them into its own. A set that had no step
+    // contributes with weight 0.
+    constexpr int kValues = 18;
+    __syncthreads();
+    float* other = reinterpret_cast<float*>(smem) + 64 * kValues * w + lane;
+    if (kg == 1) {
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) other[64 * (4 * u + e)] = acc[u][e];
+      other[64 * 16] = kg < steps ? m : -INFINITY;
+      other[64 * 17] = lacc[0];
+    }
+    __syncthreads();
+    if (kg == 1) return;
+    const float mo = other[64 * 16], mn = fmaxf(m, mo);
+    const float a0 = exp2_fast((m - mn) * kScoreToLog2), a1 = exp2_fast((mo - mn) * kScoreToLog2);
+    lacc[0] = fmaf(other[64 * 17], a1, lacc[0] * a0);
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) acc[u][e] = fmaf(other[64 * (4 * u + e)], a1, acc[u][e] * a0);
   }
 
   // lane (c, g) of tile u holds O^T[dims 16u + 4g .. + 3][position c]; every row of lacc
@@ -249,8 +325,14 @@ extern "C" int pc_prefill_attention(void* out, const void* query, const void* ke
   if (!out || !query || !key || !value) return set_error(PC_ERR_ARGUMENT, "null pointer");
   if (!aligned(out, 16) || !aligned(query, 16) || !aligned(key, 16) || !aligned(value, 16))
     return set_error(PC_ERR_ARGUMENT, "buffers must be 16-byte aligned");
-  const unsigned grid = static_cast<unsigned>((tokens + kBlock - 1) / kBlock) * kKVHeads;
-  hipLaunchKernelGGL(prefill_attention_kernel, dim3(grid), dim3(kThreads), 0, static_cast<hipStream_t>(stream),
+  // Two key sets while their workgroups (64 KiB of LDS, two per CU) run at once, above the 128
+  // tokens (two steps) where the merge costs more than the shorter chain saves: 3.8 against
+  // 4.1 us at 128 tokens, 5.1 / 5.1 at 256, 6.1 / 5.7 at 333, 12.3 / 10.6 at 1024, 15.3 / 15.3
+  // at 1280, 26.5 / 29.6 at 2048.
+  const unsigned grid = static_cast<unsigned>((tokens + kBlock - 1) / kBlock) * kPerBlock;
+  const bool split = tokens > 128 && grid <= 2 * kSnake;
+  auto kernel = split ? prefill_attention_kernel<2> : prefill_attention_kernel<1>;
+  hipLaunchKernelGGL(kernel, dim3(grid), dim3(64 * kHeads * (split ? 2 : 1)), 0, static_cast<hipStream_t>(stream),
                      static_cast<const _Float16*>(query), static_cast<const _Float16*>(key),
                      static_cast<const _Float16*>(value), static_cast<int>(tokens), static_cast<_Float16*>(out));
   return check_launch("prefill_attention");

@@ -674,6 +674,51 @@ def test_prefill_attention_sharp_and_known_answers(device):
     assert torch.all(out.cpu() == 0.375)
 
 
+def _causal_fp64_on(query, key, value):
+    """_causal_fp64 on the inputs' device, one kv head at a time (long prompts)."""
+    tokens = query.shape[0]
+    mask = ~torch.ones(tokens, tokens, dtype=torch.bool, device=query.device).tril()
+    out = torch.empty(query.shape, dtype=torch.float64, device=query.device)
+    for h in range(32):
+        scores = (query[:, h].double() @ key[:, h // 8].double().t().contiguous() / 8).masked_fill(mask, float("-inf"))
+        out[:, h] = scores.softmax(-1) @ value[:, h // 8].double()
+    return out
+
+
+@pytest.mark.parametrize("sharp", [False, True])
+@pytest.mark.parametrize("tokens", [112, 128, 129, 193, 1023, 1024, 1025, 2047, 4100])
+def test_prefill_attention_at_the_dispatch_edges(device, tokens, sharp):
+    """Both forms of the kernel (one and two key sets) on either side of the sizes where they
+    change, a last chunk of workgroups that is partly filled, and more than eight chunks;
+    unit and +-1000-scale scores, against FP64 within the kernel's 2e-3."""
+    gen = torch.Generator(device=device).manual_seed(tokens + sharp)
+    factor = 30 if sharp else 1
+    query = (torch.randn(tokens, 32, 64, device=device, generator=gen) * factor).half()
+    key = (torch.randn(tokens, 4, 64, device=device, generator=gen) * factor).half()
+    value = torch.randn(tokens, 4, 64, dtype=torch.float16, device=device, generator=gen)
+    out = torch.full((tokens + 16, 32, 64), 7.0, dtype=torch.float16, device=device)
+    _hip.prefill_attention(out[:tokens], query, key, value)
+    torch.cuda.synchronize()
+    assert torch.all(out[tokens:] == 7.0)
+    torch.testing.assert_close(out[:tokens].double(), _causal_fp64_on(query, key, value), atol=2e-3, rtol=2e-3)
+
+
+@pytest.mark.parametrize("tokens", [100, 300, 1100])
+def test_prefill_attention_with_infinite_keys(device, tokens):
+    """Keys of -inf against positive queries score -inf and weigh nothing, also where they fill
+    whole steps of 64 keys of either key set."""
+    gen = torch.Generator(device=device).manual_seed(tokens)
+    query = torch.rand(tokens, 32, 64, device=device, generator=gen).add_(0.1).half()
+    key = torch.randn(tokens, 4, 64, dtype=torch.float16, device=device, generator=gen)
+    value = torch.randn(tokens, 4, 64, dtype=torch.float16, device=device, generator=gen)
+    key[1:80] = float("-inf")
+    key[128:256] = float("-inf")
+    out = torch.empty(tokens, 32, 64, dtype=torch.float16, device=device)
+    _hip.prefill_attention(out, query, key, value)
+    torch.cuda.synchronize()
+    torch.testing.assert_close(out.double(), _causal_fp64_on(query, key, value), atol=2e-3, rtol=2e-3)
+
+
 def test_prefill_attention_rejects_bad_arguments(device):
     lib = _hip.load()
     buf = torch.empty(64, dtype=torch.float16, device=device)
