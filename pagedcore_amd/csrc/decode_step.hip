@@ -15,6 +15,8 @@
 #include <math.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #include "pagedcore_hip.h"
 #include "pc_internal.h"
 
@@ -36,7 +38,8 @@ constexpr int kHalfDim = kHeadDim / 2;                 // 32 rotation frequencie
 constexpr int64_t kRowElems = kKVHeads * kHeadDim;     // 256 fp16 per pool token row
 constexpr int kQElems = kQHeads * kHeadDim;            // 2048
 constexpr int kQkvElems = kQElems + 2 * kRowElems;     // 2560: q | k | v of one token
-constexpr int kRopeThreads = 192;                      // 128 q tasks, 16 k tasks, 32 v tasks
+constexpr int kRopeTasks = 160;                        // 128 of q, 16 of k, 16 of v
+constexpr int kRopeThreads = 192;
 constexpr int kNormThreads = 256;
 constexpr int kNormMaxChunks = 4;                      // rows of up to 4 * 256 * 8 = 8192
 constexpr int kSiluThreads = 256;
@@ -45,75 +48,96 @@ __device__ __forceinline__ _Float16 round_h(float x) { return static_cast<_Float
 
 typedef float float4_t __attribute__((ext_vector_type(4)));
 
-constexpr int kUnrolledSplits = 8;  // split counts up to this load all their parts at once
+// What bounds the two kernels below at decode sizes is the number of dependent memory round
+// trips (each about 0.6-1 us: their inputs were just written on other XCDs), so every load that
+// does not depend on another is issued before the first wait. The split count is a template
+// argument for the counts a decode step uses: 2 splits then load 2 parts (a form unrolled to 8
+// that reloaded split 0 for the missing ones took the L1 four times as long).
 
-// fp16(sum over the splits of parts[s * split_stride + offset + 0..7]), added in split order.
-// Up to kUnrolledSplits splits, every load is issued before the first add (one memory round
-// trip, not one per split); a split past `splits` reloads split 0 and is not added.
-__device__ __forceinline__ half8_t sum_parts8(const float* parts, int64_t offset, int splits, int64_t split_stride) {
-  float4_t lo, hi;
-  if (splits <= kUnrolledSplits) {
-    float4_t l[kUnrolledSplits], h[kUnrolledSplits];
-#pragma unroll
-    for (int s = 0; s < kUnrolledSplits; ++s) {
-      const float* p = parts + (s < splits ? s : 0) * split_stride + offset;
-      l[s] = *reinterpret_cast<const float4_t*>(p);
-      h[s] = *reinterpret_cast<const float4_t*>(p + 4);
-    }
-    lo = l[0];
-    hi = h[0];
-#pragma unroll
-    for (int s = 1; s < kUnrolledSplits; ++s) {
-      lo = s < splits ? lo + l[s] : lo;
-      hi = s < splits ? hi + h[s] : hi;
-    }
+constexpr int kFp16Input = 0;     // the projection is an fp16 row
+constexpr int kAnySplits = -1;    // a split count without its own instance
+
+// 8 consecutive columns of a projection: the fp16 values, or the parts that make them.
+template <int SPLITS>
+struct Chunk8 {
+  float4_t lo[SPLITS > 0 ? SPLITS : 1], hi[SPLITS > 0 ? SPLITS : 1];
+  half8_t value;
+};
+
+// Issues the chunk's loads: SPLITS fp32 parts at `offset` + s * stride of `input`, or its fp16 chunk.
+template <int SPLITS>
+__device__ __forceinline__ Chunk8<SPLITS> load8(const void* input, int64_t offset, int64_t stride) {
+  Chunk8<SPLITS> c;
+  if constexpr (SPLITS == kFp16Input) {
+    c.value = *reinterpret_cast<const half8_t*>(static_cast<const _Float16*>(input) + offset);
   } else {
-    lo = *reinterpret_cast<const float4_t*>(parts + offset);
-    hi = *reinterpret_cast<const float4_t*>(parts + offset + 4);
-    for (int s = 1; s < splits; ++s) {
-      const float* p = parts + s * split_stride + offset;
-      lo += *reinterpret_cast<const float4_t*>(p);
-      hi += *reinterpret_cast<const float4_t*>(p + 4);
+    const float* parts = static_cast<const float*>(input);
+#pragma unroll
+    for (int s = 0; s < (SPLITS > 0 ? SPLITS : 1); ++s) {
+      c.lo[s] = *reinterpret_cast<const float4_t*>(parts + s * stride + offset);
+      c.hi[s] = *reinterpret_cast<const float4_t*>(parts + s * stride + offset + 4);
     }
   }
-  half8_t out;
+  return c;
+}
+
+// fp16(sum of the parts), added in split order.
+template <int SPLITS>
+__device__ __forceinline__ half8_t value8(const Chunk8<SPLITS>& c, const void* input, int64_t offset, int64_t stride,
+                                          int splits) {
+  if constexpr (SPLITS == kFp16Input) {
+    return c.value;
+  } else {
+    float4_t lo = c.lo[0], hi = c.hi[0];
+    if constexpr (SPLITS == kAnySplits) {
+      const float* parts = static_cast<const float*>(input);
+      for (int s = 1; s < splits; ++s) {
+        lo += *reinterpret_cast<const float4_t*>(parts + s * stride + offset);
+        hi += *reinterpret_cast<const float4_t*>(parts + s * stride + offset + 4);
+      }
+    } else {
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    out[i] = round_h(lo[i]);
-    out[i + 4] = round_h(hi[i]);
+      for (int s = 1; s < SPLITS; ++s) {
+        lo += c.lo[s];
+        hi += c.hi[s];
+      }
+    }
+    half8_t out;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      out[i] = round_h(lo[i]);
+      out[i + 4] = round_h(hi[i]);
+    }
+    return out;
   }
-  return out;
+}
+
+// Calls f(integral_constant) with the instance for a split count (kFp16Input: no parts).
+template <typename F>
+void with_splits(bool fp16, int32_t splits, F&& f) {
+  if (fp16) f(std::integral_constant<int, kFp16Input>{});
+  else if (splits == 1) f(std::integral_constant<int, 1>{});
+  else if (splits == 2) f(std::integral_constant<int, 2>{});
+  else if (splits == 4) f(std::integral_constant<int, 4>{});
+  else if (splits == 8) f(std::integral_constant<int, 8>{});
+  else f(std::integral_constant<int, kAnySplits>{});
 }
 
 // ---------------------------------------------------------------------------------------
 // RoPE + KV append.
 //
-// One workgroup per token row t. Task layout (one 16 B chunk pair each):
-//   threads   0..127  q head tid / 4, dims [8c, 8c + 8) with their partners 32 further on
-//   threads 128..143  k head (tid - 128) / 4, same dims
-//   threads 144..175  v dims [8j, 8j + 8) over the 4 heads' 256 values, copied unrotated
+// One workgroup per token row t. Every thread owns a task of two 16 B chunks 32 dims apart:
+//   threads   0..127  q head tid / 4, dims [8c, 8c + 8) with their partners
+//   threads 128..143  k head (tid - 128) / 4, the same dims
+//   threads 144..159  v head (tid - 144) / 4, the same dims, not rotated
+// (threads 160..191 repeat the last task and store nothing). Two memory round trips: position,
+// slot and the projections together, then the table row of the position; six, one after the
+// other, took 5.2 us a launch at 37 rows and 4.8 at one (22 layers of rope and q|k|v at 37 rows
+// 419 -> 338 us).
 // The reference rotation (dense.py:56-59) is x * cos + cat(-x2, x1) * sin with cos/sin the
 // fp16 tables of the position; for d < 32 that is x[d] * c[d] + (-x[d + 32]) * s[d], for
 // d >= 32 x[d] * c[d - 32] + x[d - 32] * s[d - 32], each product and the sum rounded to fp16.
 // ---------------------------------------------------------------------------------------
-
-struct RopeArgs {
-  _Float16* query_out;        // [T][32][64]
-  _Float16* key_out;          // [T][4][64] or null
-  _Float16* value_out;        // [T][4][64] or null
-  const _Float16* qkv;        // [T][qkv_stride]: q (2048) | k (256) | v (256); or null and
-  const float* qkv_parts;     // [splits][T][2560] fp32 partial sums of the same columns
-  int32_t splits;
-  const int64_t* positions;   // [T]
-  const _Float16* rope;       // [rope_positions][2][32]: cos, then sin
-  _Float16* pool;             // or null
-  const int64_t* slot_mapping;  // [T] or null
-  int64_t qkv_stride;         // qkv's row stride, or qkv_parts' split stride (T * 2560)
-  int64_t slot_limit;         // num_blocks * 16
-  int64_t kind_elems;         // num_blocks * 16 * 256: one (layer, kind) plane
-  int32_t layer;
-  int32_t rope_positions;
-};
 
 __device__ __forceinline__ void rotate_pair(half8_t& lo, half8_t& hi, const half8_t c, const half8_t s) {
 #pragma clang fp contract(off)
@@ -136,84 +160,61 @@ __device__ __forceinline__ void rotate_pair(half8_t& lo, half8_t& hi, const half
   hi = out_hi;
 }
 
-// 8 columns of token t's q | k | v row, from the fp16 row or the partial sums.
-__device__ __forceinline__ half8_t load_qkv8(const RopeArgs& a, int64_t t, int col) {
-  if (a.qkv_parts != nullptr) return sum_parts8(a.qkv_parts, t * kQkvElems + col, a.splits, a.qkv_stride);
-  return *reinterpret_cast<const half8_t*>(a.qkv + t * a.qkv_stride + col);
-}
-
-// Scalar parameters, those the first loads need leading (the compiler preloads the leading
-// 56 bytes into SGPRs at wave launch: no kernel-argument round trip before them).
+// qkv: fp16 rows of stride qkv_stride (SPLITS kFp16Input), or fp32 parts [splits][T][2560] of
+// split stride qkv_stride. Scalar parameters, those the first loads need leading (the compiler
+// preloads the leading 64 bytes into SGPRs at wave launch: no kernel-argument round trip
+// before them).
+template <int SPLITS>
 __global__ __launch_bounds__(kRopeThreads) void rope_kv_append_kernel(
-    const int64_t* positions, const float* qkv_parts, const _Float16* qkv, int64_t qkv_stride, const _Float16* rope,
-    const int64_t* slot_mapping, int32_t splits, int32_t rope_positions, _Float16* pool, int64_t slot_limit,
-    int64_t kind_elems, _Float16* query_out, _Float16* key_out, _Float16* value_out, int32_t layer) {
-  RopeArgs a;
-  a.query_out = query_out;
-  a.key_out = key_out;
-  a.value_out = value_out;
-  a.qkv = qkv;
-  a.qkv_parts = qkv_parts;
-  a.splits = splits;
-  a.positions = positions;
-  a.rope = rope;
-  a.pool = pool;
-  a.slot_mapping = slot_mapping;
-  a.qkv_stride = qkv_stride;
-  a.slot_limit = slot_limit;
-  a.kind_elems = kind_elems;
-  a.layer = layer;
-  a.rope_positions = rope_positions;
+    const int64_t* positions, const int64_t* slot_mapping, const void* qkv, int64_t qkv_stride, const _Float16* rope,
+    _Float16* query_out, int32_t splits, int32_t rope_positions, _Float16* layer_pool, int64_t kind_elems,
+    _Float16* key_out, _Float16* value_out) {
   const int64_t t = blockIdx.x;
   const int tid = threadIdx.x;
-  const int64_t position = a.positions[t];
-  const bool valid_position = position >= 0 && position < a.rope_positions;
-  int64_t slot = -1;
-  if (a.pool != nullptr && a.slot_mapping != nullptr) {
-    slot = a.slot_mapping[t];
-    if (slot >= a.slot_limit) slot = -1;  // outside the pool: never written
-  }
-  const int64_t pool_row = static_cast<int64_t>(a.layer) * 2 * a.kind_elems + slot * kRowElems;
+  const int task = min(tid, kRopeTasks - 1);
+  const bool is_q = task < 128, is_v = task >= 144;
+  const int index = is_q ? task : is_v ? task - 144 : task - 128;  // within its part
+  const int offset = (index >> 2) * kHeadDim + 8 * (index & 3);    // head and dims in its part
+  const int col = offset + (is_q ? 0 : is_v ? kQElems + static_cast<int>(kRowElems) : kQElems);
+  const int64_t at = SPLITS == kFp16Input ? t * qkv_stride + col : t * kQkvElems + col;
+  const Chunk8<SPLITS> first = load8<SPLITS>(qkv, at, qkv_stride);
+  const Chunk8<SPLITS> second = load8<SPLITS>(qkv, at + kHalfDim, qkv_stride);
+  const int64_t position = positions[t];
+  int64_t slot = (slot_mapping != nullptr ? slot_mapping : positions)[t];
+  // Position, slot and the remaining arguments are scalar loads: all at once here, instead of
+  // each where it is used.
+  asm volatile("" ::"s"(position), "s"(slot), "s"(layer_pool), "s"(kind_elems), "s"(key_out), "s"(value_out));
+  if (slot_mapping == nullptr || slot >= kind_elems / kRowElems) slot = -1;  // outside the pool: never written
+  const bool valid_position = position >= 0 && position < rope_positions;
+  const _Float16* table = rope + (valid_position ? position : 0) * kHeadDim + 8 * (index & 3);
+  const half8_t cs = *reinterpret_cast<const half8_t*>(table);
+  const half8_t sn = *reinterpret_cast<const half8_t*>(table + kHalfDim);
 
-  if (tid < 144) {
-    const bool is_q = tid < 128;
-    const int task = is_q ? tid : tid - 128;
-    const int head = task >> 2;
-    const int c = task & 3;
-    const int col = (is_q ? 0 : kQElems) + head * kHeadDim + 8 * c;
-    half8_t lo = load_qkv8(a, t, col);
-    half8_t hi = load_qkv8(a, t, col + kHalfDim);
-    if (valid_position) {
-      const _Float16* table = a.rope + position * kHeadDim + 8 * c;
-      const half8_t cs = *reinterpret_cast<const half8_t*>(table);
-      const half8_t sn = *reinterpret_cast<const half8_t*>(table + kHalfDim);
-      rotate_pair(lo, hi, cs, sn);
-    } else {
-      // Never reached through the host API (positions are checked there); a bad position
-      // yields NaN rows instead of a read outside the table.
-      lo = static_cast<half8_t>(__builtin_nanf16(""));
-      hi = lo;
-    }
-    if (is_q) {
-      _Float16* dst = a.query_out + t * kQElems + head * kHeadDim + 8 * c;
-      *reinterpret_cast<half8_t*>(dst) = lo;
-      *reinterpret_cast<half8_t*>(dst + kHalfDim) = hi;
-    } else {
-      const int64_t offset = head * kHeadDim + 8 * c;
-      if (a.key_out != nullptr) {
-        *reinterpret_cast<half8_t*>(a.key_out + t * kRowElems + offset) = lo;
-        *reinterpret_cast<half8_t*>(a.key_out + t * kRowElems + offset + kHalfDim) = hi;
-      }
-      if (slot >= 0 && valid_position) {
-        *reinterpret_cast<half8_t*>(a.pool + pool_row + offset) = lo;
-        *reinterpret_cast<half8_t*>(a.pool + pool_row + offset + kHalfDim) = hi;
-      }
-    }
-  } else if (tid < 176) {
-    const int j = tid - 144;
-    const half8_t v = load_qkv8(a, t, kQElems + kRowElems + 8 * j);
-    if (a.value_out != nullptr) *reinterpret_cast<half8_t*>(a.value_out + t * kRowElems + 8 * j) = v;
-    if (slot >= 0 && valid_position) *reinterpret_cast<half8_t*>(a.pool + pool_row + a.kind_elems + 8 * j) = v;
+  half8_t lo = value8<SPLITS>(first, qkv, at, qkv_stride, splits);
+  half8_t hi = value8<SPLITS>(second, qkv, at + kHalfDim, qkv_stride, splits);
+  half8_t rotated_lo = lo, rotated_hi = hi;
+  rotate_pair(rotated_lo, rotated_hi, cs, sn);  // in every lane, so that the table is not read under a branch
+  // A bad position is never reached through the host API (positions are checked there); it
+  // yields NaN rows instead of a read outside the table.
+  const half8_t nan = static_cast<half8_t>(__builtin_nanf16(""));
+  lo = is_v ? lo : valid_position ? rotated_lo : nan;
+  hi = is_v ? hi : valid_position ? rotated_hi : nan;
+  if (tid >= kRopeTasks) return;
+  if (is_q) {
+    _Float16* dst = query_out + t * kQElems + offset;
+    *reinterpret_cast<half8_t*>(dst) = lo;
+    *reinterpret_cast<half8_t*>(dst + kHalfDim) = hi;
+    return;
+  }
+  _Float16* out = is_v ? value_out : key_out;
+  if (out != nullptr) {
+    *reinterpret_cast<half8_t*>(out + t * kRowElems + offset) = lo;
+    *reinterpret_cast<half8_t*>(out + t * kRowElems + offset + kHalfDim) = hi;
+  }
+  if (slot >= 0 && valid_position) {
+    _Float16* dst = layer_pool + (is_v ? kind_elems : 0) + slot * kRowElems + offset;
+    *reinterpret_cast<half8_t*>(dst) = lo;
+    *reinterpret_cast<half8_t*>(dst + kHalfDim) = hi;
   }
 }
 
@@ -224,52 +225,66 @@ __global__ __launch_bounds__(kRopeThreads) void rope_kv_append_kernel(
 //   h   = fp16(hidden + delta)                     (only when delta is given; stored back)
 //   r   = 1 / sqrt(sum(h * h) / width + eps)       (fp32)
 //   out = fp16(weight * fp16(h * r))
+// Rows of up to 2048 (one chunk per thread) load weight, residual and every part together, with
+// no branch between them: one memory round trip (22 layers of a 7-row MLP 435 -> 414 us, of a
+// 128-row one 731 -> 708).
 // ---------------------------------------------------------------------------------------
 
-__device__ __forceinline__ float wave_sum(float x) {
-#pragma unroll
-  for (int offset = 32; offset > 0; offset >>= 1) x += __shfl_xor(x, offset, 64);
-  return x;
+template <int CTRL>
+__device__ __forceinline__ float add_dpp(float x) {
+  const int moved = __builtin_amdgcn_update_dpp(0, __float_as_int(x), CTRL, 0xf, 0xf, false);
+  return x + __int_as_float(moved);
 }
 
-// delta, when given, is fp16 [rows][width] or (delta_parts, splits) fp32 partial sums
-// [splits][rows][width], rounded to fp16 before the add. The parameters the first loads need
-// lead (they are preloaded into SGPRs).
-__global__ __launch_bounds__(kNormThreads) void add_rms_norm_kernel(_Float16* __restrict__ hidden,
-                                                                    const float* __restrict__ delta_parts,
-                                                                    const _Float16* __restrict__ delta,
-                                                                    int64_t parts_stride, int32_t splits,
-                                                                    int32_t width, float eps,
-                                                                    const _Float16* __restrict__ weight,
-                                                                    _Float16* __restrict__ out) {
+// Sum over the wave in every lane: halves, 16-lane groups, then rotations by 8, 4, 2 and 1 within
+// each group (the additions of an xor butterfly, without its LDS round trips).
+__device__ __forceinline__ float wave_sum(float x) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  x = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+  const auto q = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  x = __uint_as_float(q[0]) + __uint_as_float(q[1]);
+  x = add_dpp<0x128>(x);  // row_ror 8, 4, 2, 1
+  x = add_dpp<0x124>(x);
+  x = add_dpp<0x122>(x);
+  return add_dpp<0x121>(x);
+}
+
+// delta, when given (HAS_DELTA), is fp16 [rows][width] (SPLITS kFp16Input) or fp32 partial sums
+// [splits][rows][width], rounded to fp16 before the add. CHUNKS chunks per thread. All the
+// parameters fit the 64 bytes that are preloaded into SGPRs.
+template <int CHUNKS, bool HAS_DELTA, int SPLITS>
+__global__ __launch_bounds__(kNormThreads) void add_rms_norm_kernel(_Float16* hidden, const void* delta,
+                                                                    int64_t parts_stride, const _Float16* weight,
+                                                                    _Float16* out, int32_t splits, int32_t width,
+                                                                    float eps) {
 #pragma clang fp contract(off)
   __shared__ float wave_sums[kNormThreads / 64];
   const int64_t base = static_cast<int64_t>(blockIdx.x) * width;
   const int tid = threadIdx.x;
   const int chunks = width / 8;
-  // The weight chunks are loaded first, with the same guards as their use below, so that
-  // their round trip overlaps the residual's instead of following the reduction.
-  half8_t wt[kNormMaxChunks];
+  half8_t wt[CHUNKS], h[CHUNKS];
+  Chunk8<SPLITS> d[CHUNKS];
+  int64_t at[CHUNKS];
+  bool mine[CHUNKS];
 #pragma unroll
-  for (int k = 0; k < kNormMaxChunks; ++k) {
+  for (int k = 0; k < CHUNKS; ++k) {
     const int chunk = tid + k * kNormThreads;
-    if (chunk < chunks) wt[k] = *reinterpret_cast<const half8_t*>(weight + 8 * chunk);
+    mine[k] = chunk < chunks;
+    const int safe = mine[k] ? chunk : chunks - 1;  // threads past the row repeat its last chunk
+    at[k] = base + 8 * safe;
+    if constexpr (HAS_DELTA) d[k] = load8<SPLITS>(delta, at[k], parts_stride);
+    h[k] = *reinterpret_cast<const half8_t*>(hidden + at[k]);
+    wt[k] = *reinterpret_cast<const half8_t*>(weight + 8 * safe);
   }
-  half8_t h[kNormMaxChunks];
   float squares = 0.0f;
 #pragma unroll
-  for (int k = 0; k < kNormMaxChunks; ++k) {
-    const int chunk = tid + k * kNormThreads;
-    if (chunk < chunks) {
-      _Float16* p = hidden + base + 8 * chunk;
-      h[k] = *reinterpret_cast<const half8_t*>(p);
-      if (delta != nullptr || delta_parts != nullptr) {
-        const half8_t d = delta_parts != nullptr ? sum_parts8(delta_parts, base + 8 * chunk, splits, parts_stride)
-                                                 : *reinterpret_cast<const half8_t*>(delta + base + 8 * chunk);
+  for (int k = 0; k < CHUNKS; ++k) {
+    if constexpr (HAS_DELTA) {
+      const half8_t v = value8<SPLITS>(d[k], delta, at[k], parts_stride, splits);
 #pragma unroll
-        for (int i = 0; i < 8; ++i) h[k][i] = round_h(static_cast<float>(h[k][i]) + static_cast<float>(d[i]));
-        *reinterpret_cast<half8_t*>(p) = h[k];
-      }
+      for (int i = 0; i < 8; ++i) h[k][i] = round_h(static_cast<float>(h[k][i]) + static_cast<float>(v[i]));
+    }
+    if (mine[k]) {
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
         const float x = static_cast<float>(h[k][i]);
@@ -279,22 +294,24 @@ __global__ __launch_bounds__(kNormThreads) void add_rms_norm_kernel(_Float16* __
   }
   squares = wave_sum(squares);
   if ((tid & 63) == 0) wave_sums[tid >> 6] = squares;
+  // The barrier also orders every thread's residual loads before the first store: threads past
+  // the row read a chunk that another thread stores.
   __syncthreads();
   float total = 0.0f;
 #pragma unroll
   for (int w = 0; w < kNormThreads / 64; ++w) total += wave_sums[w];
   const float scale = 1.0f / sqrtf(total / static_cast<float>(width) + eps);
 #pragma unroll
-  for (int k = 0; k < kNormMaxChunks; ++k) {
-    const int chunk = tid + k * kNormThreads;
-    if (chunk < chunks) {
+  for (int k = 0; k < CHUNKS; ++k) {
+    if (mine[k]) {
       half8_t o;
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
         const float normalized = static_cast<float>(round_h(static_cast<float>(h[k][i]) * scale));
         o[i] = round_h(static_cast<float>(wt[k][i]) * normalized);
       }
-      *reinterpret_cast<half8_t*>(out + base + 8 * chunk) = o;
+      if constexpr (HAS_DELTA) *reinterpret_cast<half8_t*>(hidden + at[k]) = h[k];
+      *reinterpret_cast<half8_t*>(out + at[k]) = o;
     }
   }
 }
@@ -326,14 +343,6 @@ __global__ __launch_bounds__(kSiluThreads) void silu_mul_kernel(_Float16* __rest
   *reinterpret_cast<half8_t*>(out + r * width + 8 * c) = o;
 }
 
-}  // namespace
-
-extern "C" {
-
-}  // extern "C"
-
-namespace {
-
 // Shared by both RoPE entry points: exactly one of qkv / qkv_parts is given (checked by the
 // callers), with qkv_stride its row stride or split stride.
 int rope_kv_append(void* query_out, void* key_out, void* value_out, const void* qkv, const float* qkv_parts,
@@ -352,12 +361,15 @@ int rope_kv_append(void* query_out, void* key_out, void* value_out, const void* 
   if (!aligned(query_out, 16) || !aligned(qkv, 16) || !aligned(qkv_parts, 16) || !aligned(rope_table, 16) ||
       !aligned(pool, 16) || !aligned(key_out, 16) || !aligned(value_out, 16))
     return set_error(PC_ERR_ARGUMENT, "buffers must be 16-byte aligned");
-  hipLaunchKernelGGL(rope_kv_append_kernel, dim3(static_cast<uint32_t>(num_tokens)), dim3(kRopeThreads), 0,
-                     static_cast<hipStream_t>(stream), positions, qkv_parts, static_cast<const _Float16*>(qkv),
-                     qkv_stride, static_cast<const _Float16*>(rope_table), slot_mapping, splits, rope_positions,
-                     static_cast<_Float16*>(pool), pool ? num_blocks * kSlots : int64_t{0},
-                     pool ? num_blocks * kSlots * kRowElems : int64_t{0}, static_cast<_Float16*>(query_out),
-                     static_cast<_Float16*>(key_out), static_cast<_Float16*>(value_out), pool ? layer : 0);
+  const int64_t kind_elems = pool ? num_blocks * kSlots * kRowElems : 0;
+  _Float16* layer_pool = pool ? static_cast<_Float16*>(pool) + static_cast<int64_t>(layer) * 2 * kind_elems : nullptr;
+  with_splits(qkv_parts == nullptr, splits, [&](auto instance) {
+    hipLaunchKernelGGL(rope_kv_append_kernel<decltype(instance)::value>, dim3(static_cast<uint32_t>(num_tokens)),
+                       dim3(kRopeThreads), 0, static_cast<hipStream_t>(stream), positions, slot_mapping,
+                       qkv_parts ? static_cast<const void*>(qkv_parts) : qkv, qkv_stride,
+                       static_cast<const _Float16*>(rope_table), static_cast<_Float16*>(query_out), splits, rope_positions,
+                       layer_pool, kind_elems, static_cast<_Float16*>(key_out), static_cast<_Float16*>(value_out));
+  });
   return check_launch("rope_kv_append");
 }
 
@@ -373,10 +385,22 @@ int add_rms_norm(void* out, void* hidden, const void* delta, const float* delta_
   if (!aligned(out, 16) || !aligned(hidden, 16) || !aligned(delta, 16) || !aligned(delta_parts, 16) ||
       !aligned(weight, 16))
     return set_error(PC_ERR_ARGUMENT, "buffers must be 16-byte aligned");
-  hipLaunchKernelGGL(add_rms_norm_kernel, dim3(static_cast<uint32_t>(rows)), dim3(kNormThreads), 0,
-                     static_cast<hipStream_t>(stream), static_cast<_Float16*>(hidden), delta_parts,
-                     static_cast<const _Float16*>(delta), rows * width, splits, width, eps,
-                     static_cast<const _Float16*>(weight), static_cast<_Float16*>(out));
+  auto launch = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(static_cast<uint32_t>(rows)), dim3(kNormThreads), 0, static_cast<hipStream_t>(stream),
+                       static_cast<_Float16*>(hidden), delta_parts ? static_cast<const void*>(delta_parts) : delta,
+                       rows * width, static_cast<const _Float16*>(weight), static_cast<_Float16*>(out), splits, width, eps);
+  };
+  const bool one_chunk = width <= kNormThreads * 8;
+  if (delta == nullptr && delta_parts == nullptr) {
+    one_chunk ? launch(add_rms_norm_kernel<1, false, kFp16Input>) : launch(add_rms_norm_kernel<kNormMaxChunks, false, kFp16Input>);
+  } else {
+    with_splits(delta_parts == nullptr, splits, [&](auto instance) {
+      constexpr int S = decltype(instance)::value;
+      // Longer rows hold every chunk's parts in registers only one split at a time.
+      if (one_chunk) launch(add_rms_norm_kernel<1, true, S>);
+      else launch(add_rms_norm_kernel<kNormMaxChunks, true, S == kFp16Input ? kFp16Input : kAnySplits>);
+    });
+  }
   return check_launch("add_rms_norm");
 }
 

@@ -286,3 +286,73 @@ def test_gemm_rows_tiles(device, m, n, k, splits):
             torch.cuda.synchronize()
             assert (fused[m * (n // 2) :] == -77.0).all()
             assert np.array_equal(_bits(fused[: m * (n // 2)]), _bits(separate.view(-1)))
+
+
+# --- the split-K consumers' instances (1, 2, 4, 8 and any other split count; row lengths) ------
+
+
+@pytest.mark.parametrize("splits", [1, 2, 3, 4, 8, 9])
+@pytest.mark.parametrize("rows,width", [(1, 8), (3, 504), (5, 2048), (2, 2056), (3, 8192)])
+def test_add_rms_norm_instances(device, rows, width, splits):
+    """Parts bit equal to the fp16 path fed their rounded sum, and that path against float64:
+    the residual exact, the output within its two fp16 roundings."""
+    gen = torch.Generator(device=device).manual_seed(rows * width + splits)
+    parts = torch.randn((splits, rows, width), device=device, generator=gen) * 0.3
+    hidden = torch.randn((rows, width), device=device, generator=gen).half()
+    weight = (1 + 0.1 * torch.randn(width, device=device, generator=gen)).half()
+    delta = _sum_in_split_order(parts)
+    results = []
+    for given in (parts, delta, None):
+        guard = torch.full((2, rows * width + 32), 7.0, dtype=torch.float16, device=device)
+        h, out = guard[0, : rows * width].view(rows, width), guard[1, : rows * width].view(rows, width)
+        h.copy_(hidden)
+        (_hip.add_rms_norm_parts if given is parts else _hip.add_rms_norm)(out, h, given, weight, dec.RMS_EPS)
+        torch.cuda.synchronize()
+        assert (guard[:, rows * width :] == 7.0).all()
+        results.append((h, out))
+        summed = hidden if given is None else (hidden.float() + delta.float()).half()
+        assert torch.equal(h, summed)
+        exact = summed.double() * torch.rsqrt(summed.double().square().mean(-1, keepdim=True) + dec.RMS_EPS) * weight.double()
+        # two roundings to fp16 (the second may be of a value rounded first), fp32 elsewhere
+        assert ((out.double() - exact).abs() <= exact.abs() * (2.0**-10 + 2.0**-18) + 2.0**-23).all()
+    assert np.array_equal(_bits(results[0][0]), _bits(results[1][0]))
+    assert np.array_equal(_bits(results[0][1]), _bits(results[1][1]))
+
+
+@pytest.mark.parametrize("splits", [1, 2, 3, 4, 8, 9])
+@pytest.mark.parametrize("outputs", ["pool", "contiguous", "both"])
+def test_rope_kv_append_instances(device, splits, outputs):
+    """Parts bit equal to the fp16 path (checked against the oracle elsewhere) with each set of
+    outputs; slots of -1 and past the pool, and their neighbours' rows, stay untouched."""
+    tokens, blocks = 9, 4
+    gen = torch.Generator(device=device).manual_seed(splits)
+    parts = torch.randn((splits, tokens, 2560), device=device, generator=gen) * 0.5
+    positions = torch.randint(0, 2048, (tokens,), device=device, generator=gen)
+    slots = torch.randperm(blocks * 16, device=device, generator=gen)[:tokens]
+    slots[2], slots[5] = -1, blocks * 16
+    table = dec.rope_table(device)
+    results = []
+    for use_parts in (False, True):
+        pool = torch.full((22, 2, blocks, 16, 4, 64), 7.0, dtype=torch.float16, device=device)
+        query = torch.empty(tokens, 32, 64, dtype=torch.float16, device=device)
+        keys = torch.full((tokens, 4, 64), 7.0, dtype=torch.float16, device=device)
+        values = torch.full_like(keys, 7.0)
+        given = {} if outputs == "pool" else {"key_out": keys, "value_out": values}
+        if outputs != "contiguous":
+            given.update(pool=pool, layer=21, slot_mapping=slots)
+        if use_parts:
+            _hip.rope_kv_append_parts(query, parts, positions, table, **given)
+        else:
+            _hip.rope_kv_append(query, _sum_in_split_order(parts), positions, table, **given)
+        torch.cuda.synchronize()
+        results.append((query, keys, values, pool))
+        written = torch.zeros(blocks * 16, dtype=torch.bool, device=device)
+        if outputs != "contiguous":
+            written[slots[(slots >= 0) & (slots < blocks * 16)]] = True
+        assert (pool[:21] == 7.0).all() and (pool[21].view(2, -1, 4, 64)[:, ~written] == 7.0).all()
+        if outputs == "both":
+            kept = (slots >= 0) & (slots < blocks * 16)
+            assert torch.equal(pool[21, 0].view(-1, 4, 64)[slots[kept]], keys[kept])
+            assert torch.equal(pool[21, 1].view(-1, 4, 64)[slots[kept]], values[kept])
+    for a, b in zip(*results):
+        assert np.array_equal(_bits(a), _bits(b))
