@@ -303,6 +303,23 @@ int pc_gemm_rows(void* out, const void* x, const void* w, int32_t m, int32_t n, 
                  int32_t epilogue, void* stream);
 
 /*
+ * The q|k|v projection of up to 65536 token rows with pc_rope_kv_append as its epilogue: one
+ * launch, no q|k|v matrix in memory.
+ *
+ * Replaces the q, k and v torch.nn.functional.linear calls, apply_rope and the cache write of a
+ * layer (reference src/pagedcore/dense.py:33-61 and 91-104 via src/pagedcore/decoder.py:113-135
+ * and :173-187). fp32 accumulation in one order for every m up to 288, one rounding to fp16,
+ * then the computation of pc_rope_kv_append.
+ *
+ *   x  [m][k] fp16, w [2560][k] fp16 (the stacked q, k and v weights), k a multiple of 64 up to
+ *   2^18, m * k up to 2^31; the other arguments are those of pc_rope_kv_append for m tokens. No
+ *   output may overlap x or w.
+ */
+int pc_qkv_rope_append(void* query_out, void* key_out, void* value_out, const void* x, const void* w, int32_t m, int32_t k,
+                       const int64_t* positions, const void* rope_table, int32_t rope_positions, void* pool,
+                       int64_t num_blocks, int32_t layer, const int64_t* slot_mapping, void* stream);
+
+/*
  * Causal attention of one prompt over its contiguous K/V (the prefill of one sequence).
  *
  * Replaces the prompt's dense_attention (reference src/pagedcore/dense.py:69-81, called by

@@ -113,6 +113,8 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.pc_prefill_attention.argtypes = [_p, _p, _p, _p, _i32, _p]
     lib.pc_rope_kv_append_parts.restype = ctypes.c_int
     lib.pc_rope_kv_append_parts.argtypes = [_p, _p, _p, _p, _i32, _p, _p, _i32, _p, _i64, _i32, _p, _i64, _p]
+    lib.pc_qkv_rope_append.restype = ctypes.c_int
+    lib.pc_qkv_rope_append.argtypes = [_p, _p, _p, _p, _p, _i32, _i32, _p, _p, _i32, _p, _i64, _i32, _p, _p]
     lib.pc_add_rms_norm_parts.restype = ctypes.c_int
     lib.pc_add_rms_norm_parts.argtypes = [_p, _p, _p, _i32, _p, _i64, _i32, ctypes.c_float, _p]
     lib.pc_gemm_m128.restype = ctypes.c_int
@@ -442,6 +444,47 @@ def rope_kv_append_parts(
         _stream(qkv_parts.device),
     )
     _check(lib, "pc_rope_kv_append_parts", status)
+
+
+def qkv_rope_append(
+    query_out: Tensor,
+    x: Tensor,
+    w: Tensor,
+    positions: Tensor,
+    rope_table: Tensor,
+    *,
+    key_out: Optional[Tensor] = None,
+    value_out: Optional[Tensor] = None,
+    pool: Optional[Tensor] = None,
+    layer: int = 0,
+    slot_mapping: Optional[Tensor] = None,
+) -> None:
+    """rope_kv_append of the q | k | v projection x @ w.T, in one launch (pc_qkv_rope_append): x
+    contiguous fp16 [tokens, k], w contiguous fp16 [2560, k]; the outputs of rope_kv_append."""
+    lib = load()
+    m, k = x.shape
+    if x.dtype != torch.float16 or w.dtype != torch.float16 or tuple(w.shape) != (2560, k):
+        raise HipExtensionError("x and w must be fp16 [tokens, k] and [2560, k]")
+    if not (x.is_contiguous() and w.is_contiguous()):
+        raise HipExtensionError("x and w must be contiguous")
+    status = lib.pc_qkv_rope_append(
+        query_out.data_ptr(),
+        _ptr(key_out),
+        _ptr(value_out),
+        x.data_ptr(),
+        w.data_ptr(),
+        m,
+        k,
+        positions.data_ptr(),
+        rope_table.data_ptr(),
+        rope_table.shape[0],
+        _ptr(pool),
+        pool.shape[2] if pool is not None else 0,
+        layer,
+        _ptr(slot_mapping),
+        _stream(x.device),
+    )
+    _check(lib, "pc_qkv_rope_append", status)
 
 
 def add_rms_norm_parts(out: Tensor, hidden: Tensor, delta_parts: Tensor, weight: Tensor, eps: float = 1e-5) -> None:

@@ -19,9 +19,11 @@
 
 #include "pagedcore_hip.h"
 #include "pc_internal.h"
+#include "rope_device.h"
 
 namespace {
 
+using namespace rope_device;
 using pc_internal::aligned;
 using pc_internal::check_launch;
 using pc_internal::ok;
@@ -29,15 +31,6 @@ using pc_internal::set_error;
 
 typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
 
-constexpr int kLayers = 22;
-constexpr int kSlots = 16;
-constexpr int kKVHeads = 4;
-constexpr int kQHeads = 32;
-constexpr int kHeadDim = 64;
-constexpr int kHalfDim = kHeadDim / 2;                 // 32 rotation frequencies
-constexpr int64_t kRowElems = kKVHeads * kHeadDim;     // 256 fp16 per pool token row
-constexpr int kQElems = kQHeads * kHeadDim;            // 2048
-constexpr int kQkvElems = kQElems + 2 * kRowElems;     // 2560: q | k | v of one token
 constexpr int kRopeTasks = 160;                        // 128 of q, 16 of k, 16 of v
 constexpr int kRopeThreads = 192;
 constexpr int kNormThreads = 256;
@@ -134,31 +127,7 @@ void with_splits(bool fp16, int32_t splits, F&& f) {
 // slot and the projections together, then the table row of the position; six, one after the
 // other, took 5.2 us a launch at 37 rows and 4.8 at one (22 layers of rope and q|k|v at 37 rows
 // 419 -> 338 us).
-// The reference rotation (dense.py:56-59) is x * cos + cat(-x2, x1) * sin with cos/sin the
-// fp16 tables of the position; for d < 32 that is x[d] * c[d] + (-x[d + 32]) * s[d], for
-// d >= 32 x[d] * c[d - 32] + x[d - 32] * s[d - 32], each product and the sum rounded to fp16.
 // ---------------------------------------------------------------------------------------
-
-__device__ __forceinline__ void rotate_pair(half8_t& lo, half8_t& hi, const half8_t c, const half8_t s) {
-#pragma clang fp contract(off)
-  half8_t out_lo, out_hi;
-#pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const float x1 = static_cast<float>(lo[i]);
-    const float x2 = static_cast<float>(hi[i]);
-    const float cf = static_cast<float>(c[i]);
-    const float sf = static_cast<float>(s[i]);
-    const float a1 = static_cast<float>(round_h(x1 * cf));
-    // fp16(-a * b) == -fp16(a * b): round-to-nearest-even is symmetric.
-    const float b1 = static_cast<float>(-round_h(x2 * sf));
-    const float a2 = static_cast<float>(round_h(x2 * cf));
-    const float b2 = static_cast<float>(round_h(x1 * sf));
-    out_lo[i] = round_h(a1 + b1);
-    out_hi[i] = round_h(a2 + b2);
-  }
-  lo = out_lo;
-  hi = out_hi;
-}
 
 // qkv: fp16 rows of stride qkv_stride (SPLITS kFp16Input), or fp32 parts [splits][T][2560] of
 // split stride qkv_stride. Scalar parameters, those the first loads need leading (the compiler
@@ -193,7 +162,7 @@ __global__ __launch_bounds__(kRopeThreads) void rope_kv_append_kernel(
   half8_t lo = value8<SPLITS>(first, qkv, at, qkv_stride, splits);
   half8_t hi = value8<SPLITS>(second, qkv, at + kHalfDim, qkv_stride, splits);
   half8_t rotated_lo = lo, rotated_hi = hi;
-  rotate_pair(rotated_lo, rotated_hi, cs, sn);  // in every lane, so that the table is not read under a branch
+  rotate_pair<8>(rotated_lo, rotated_hi, cs, sn);  // in every lane, so that the table is not read under a branch
   // A bad position is never reached through the host API (positions are checked there); it
   // yields NaN rows instead of a read outside the table.
   const half8_t nan = static_cast<half8_t>(__builtin_nanf16(""));

@@ -12,6 +12,7 @@
 
 #include "pagedcore_hip.h"
 #include "pc_internal.h"
+#include "rope_device.h"
 
 namespace gemm_device {
 
@@ -19,7 +20,14 @@ typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
 typedef _Float16 half4_t __attribute__((ext_vector_type(4)));
 typedef float float4_t __attribute__((ext_vector_type(4)));
 
-enum Epilogue : int32_t { kPartials = PC_GEMM_PARTIALS, kHalf = PC_GEMM_HALF, kSwiGLU = PC_GEMM_SWIGLU };
+// kRope: the q|k|v projection rotated and written where pc_rope_kv_append writes it.
+enum Epilogue : int32_t { kPartials = PC_GEMM_PARTIALS, kHalf = PC_GEMM_HALF, kSwiGLU = PC_GEMM_SWIGLU, kRope = 3 };
+// The epilogues whose tiles hold pairs of W rows: gate and up, or a head's d and d + 32.
+constexpr bool paired(Epilogue e) { return e == kSwiGLU || e == kRope; }
+template <Epilogue E>
+struct OutOf { typedef void* type; };
+template <>
+struct OutOf<kRope> { typedef rope_device::RopeOut type; };
 
 __device__ __forceinline__ __attribute__((address_space(3))) void* lds_ptr(char* p) {
   return (__attribute__((address_space(3))) void*)(p);
@@ -69,6 +77,17 @@ inline int raise_lds_limit(const void* kernel, int bytes, std::atomic<uint64_t>&
   done.fetch_or(bit, std::memory_order_acq_rel);
   return PC_OK;
 }
+
+// A q|k|v projection with the RoPE epilogue (x [m][k], w [2560][k]).
+struct QkvArgs {
+  const _Float16* x;
+  const _Float16* w;
+  int m, k;
+  const int64_t* positions;
+  const int64_t* slots;  // null: no pool
+  rope_device::RopeOut out;
+};
+int launch_qkv_rows(const QkvArgs& a, hipStream_t s);  // the tiles of a prompt's rows
 
 }  // namespace gemm_device
 

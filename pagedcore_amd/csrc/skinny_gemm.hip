@@ -15,7 +15,12 @@
 // v_mfma_f32_16x16x32_f16 with W as the A operand (16 weight rows) and X as the B operand
 // (16 activation rows), so each lane ends with 4 consecutive output columns of one row.
 //
-// That form (gemm_m128_kernel) is for many rows: its X ring has 128 rows whatever m is. Up to
+// pc_qkv_rope_append is here too: the q|k|v projection whose epilogue rotates q and k and writes
+// them and v where pc_rope_kv_append does (pairs of a head's columns d and d + 32 in one tile, no
+// split-K, so that a workgroup holds final sums). A launch, a round trip of the partials and
+// a kernel of a few kilobytes per row less in every layer.
+//
+// The form above (gemm_m128_kernel) is for many rows: its X ring has 128 rows whatever m is. Up to
 // 64 rows, and where it leaves CUs idle, gemm_stream_kernel takes over (see there).
 //
 // Epilogues: fp32 partials [splits][m][n]; fp16 [m][n] (one split); or SwiGLU (one split):
@@ -28,11 +33,13 @@
 namespace {
 
 using namespace gemm_device;
+using namespace rope_device;
 using pc_internal::aligned;
 using pc_internal::check_launch;
 using pc_internal::set_error;
 
 constexpr int kMaxRows = 128;
+constexpr int kMaxQkvK = 1 << 18;  // 2560 rows of W within 32-bit offsets
 constexpr int kSwiGLUHalf = 32;  // gate (and up) rows per SwiGLU tile
 
 struct GemmArgs {
@@ -244,10 +251,12 @@ struct StreamShape {
 
 template <int MT, int NT, int WAVES, int D, Epilogue E>
 __global__ __launch_bounds__(64 * WAVES) void gemm_stream_kernel(const _Float16* x, const _Float16* w, int m, int n,
-                                                                 int k, int ksplit, int tiles, int mtiles, void* out) {
+                                                                 int k, int ksplit, int tiles, int mtiles,
+                                                                 const int64_t* positions, const int64_t* slots,
+                                                                 typename OutOf<E>::type out) {
   using S = StreamShape<MT, NT, WAVES, D>;
   constexpr int kRowsX = 16 * MT, kXBytes = 2048 * MT;
-  constexpr int kCols = E == kSwiGLU ? 8 * NT : 16 * NT;  // output columns per tile (SwiGLU: gate rows)
+  constexpr int kCols = paired(E) ? 8 * NT : 16 * NT;  // output columns per tile (pairs of them)
   extern __shared__ __attribute__((aligned(16))) char smem[];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
@@ -261,7 +270,7 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_stream_kernel(const _Float16*
   }
   const int tile = id % tiles, split = id / tiles;
   if (split * ksplit >= k) return;  // the grid is rounded up to 8 tiles
-  const int limit = E == kSwiGLU ? n / 2 : n;
+  const int limit = paired(E) ? n / 2 : n;
   const int units = ksplit / 64;
   const int mine = (units - wave + WAVES - 1) / WAVES;
 
@@ -280,13 +289,28 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_stream_kernel(const _Float16*
     if constexpr (E == kSwiGLU) {
       const int last = limit - 1 - kCols * tile;
       woff[i] = (r < kCols ? min(r, last) : limit + min(r - kCols, last)) * line + chunk;
+    } else if constexpr (E == kRope) {
+      const int first = pair_row(kCols * tile);  // a tile's pairs are consecutive rows of one head
+      woff[i] = (first + (r < kCols ? r : kHalfDim + r - kCols)) * line + chunk;
     } else {
       woff[i] = min(r, limit - 1 - kCols * tile) * line + chunk;
     }
   }
+  // RoPE: thread e ends with quad e % Q of row e / Q of the tile (one each at most). Its position
+  // and slot are loaded before the stream's first unit and the table values behind it, so that
+  // the stream hides both round trips (loads return in order: an older one in flight only
+  // makes the waits below longer).
+  constexpr int Q = kCols / 4;  // groups of four output columns
+  static_assert(E != kRope || (kHalfDim % kCols == 0 && Q * kRowsX <= 64 * WAVES), "one quad of one head per thread");
+  int64_t position = 0, slot = 0;
+  if constexpr (E == kRope) {
+    const int row = min(kRowsX * mtile + static_cast<int>(threadIdx.x) / Q, m - 1);
+    position = positions[row];
+    slot = (slots != nullptr ? slots : positions)[row];
+  }
   const int64_t k0 = static_cast<int64_t>(split) * ksplit + 64 * wave;
   const char* xbase = reinterpret_cast<const char*>(x + static_cast<int64_t>(kRowsX) * mtile * k + k0);
-  const char* wbase = reinterpret_cast<const char*>(w + static_cast<int64_t>(kCols) * tile * k + k0);
+  const char* wbase = reinterpret_cast<const char*>(w + (E == kRope ? 0 : static_cast<int64_t>(kCols) * tile * k) + k0);
   char* const ring = smem + wave * D * S::UB;
   auto issue = [&](char* slot) {
     asm volatile("" ::: "memory");
@@ -309,6 +333,14 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_stream_kernel(const _Float16*
 #pragma unroll
   for (int t = 0; t < D; ++t) {
     if (t < mine) issue(ring + t * S::UB);
+  }
+  [[maybe_unused]] RopeRow rope{};
+  [[maybe_unused]] half4_t cs{}, sn{};
+  if constexpr (E == kRope) {
+    rope = rope_row(out, position, slot, slots != nullptr);
+    const _Float16* table = rope.table + (kCols * tile + 4 * (static_cast<int>(threadIdx.x) % Q)) % kHalfDim;
+    cs = *reinterpret_cast<const half4_t*>(table);
+    sn = *reinterpret_cast<const half4_t*>(table + kHalfDim);
   }
 
   const uint32_t ring0 = lds_offset(ring);
@@ -369,7 +401,6 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_stream_kernel(const _Float16*
 #pragma unroll
     for (int j = 0; j < MT; ++j) sums[(wave * T + i * MT + j) * 64 + lane] = acc[i][j];
   __syncthreads();
-  constexpr int Q = kCols / 4;  // groups of four output columns
   for (int e = threadIdx.x; e < Q * kRowsX; e += 64 * WAVES) {
     const int q = e % Q, r = e / Q;
     const int row = kRowsX * mtile + r, col = kCols * tile + 4 * q;
@@ -387,6 +418,15 @@ __global__ __launch_bounds__(64 * WAVES) void gemm_stream_kernel(const _Float16*
 #pragma unroll
       for (int i = 0; i < 4; ++i) o[i] = swiglu(gate[i], up[i]);
       *reinterpret_cast<half4_t*>(static_cast<_Float16*>(out) + static_cast<int64_t>(row) * limit + col) = o;
+    } else if constexpr (E == kRope) {
+      const float4_t low = total(q), high = total(Q + q);
+      half4_t lo, hi;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        lo[i] = round_h(low[i]);
+        hi[i] = round_h(high[i]);
+      }
+      store_pairs(out, rope, row, col, lo, hi, cs, sn);
     } else {
       const float4_t v = total(q);
       if constexpr (E == kHalf) {
@@ -417,20 +457,26 @@ int launch(GemmArgs a, int splits, hipStream_t s) {
 }
 
 template <int MT, int NT, int WAVES, int D, Epilogue E>
-int launch_stream(const GemmArgs& a, int splits, hipStream_t s) {
+int launch_stream(const GemmArgs& a, int splits, const int64_t* positions, const int64_t* slots,
+                  typename OutOf<E>::type out, hipStream_t s) {
   using S = StreamShape<MT, NT, WAVES, D>;
   if (a.ksplit % 64 != 0) return set_error(PC_ERR_ARGUMENT, "k per split (%d) must be a multiple of 64", a.ksplit);
   auto kernel = gemm_stream_kernel<MT, NT, WAVES, D, E>;
   static std::atomic<uint64_t> raised{0};
   if (int rc = raise_lds_limit(reinterpret_cast<const void*>(kernel), S::LDS, raised)) return rc;
-  constexpr int cols = E == kSwiGLU ? 8 * NT : 16 * NT;
-  const int tiles = ((E == kSwiGLU ? a.n / 2 : a.n) + cols - 1) / cols;
+  constexpr int cols = paired(E) ? 8 * NT : 16 * NT;
+  const int tiles = ((paired(E) ? a.n / 2 : a.n) + cols - 1) / cols;
   const int mtiles = (a.m + 16 * MT - 1) / (16 * MT);
   int64_t grid = static_cast<int64_t>(tiles) * splits;
   if (mtiles > 1) grid = (grid + 7) / 8 * 8 * mtiles;
   hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(grid)), dim3(64 * WAVES), S::LDS, s, a.x, a.w, a.m, a.n, a.k,
-                     a.ksplit, tiles, mtiles, a.out);
+                     a.ksplit, tiles, mtiles, positions, slots, out);
   return check_launch("gemm_stream");
+}
+
+template <int MT, int NT, int WAVES, int D, Epilogue E>
+int launch_stream(const GemmArgs& a, int splits, hipStream_t s) {
+  return launch_stream<MT, NT, WAVES, D, E>(a, splits, nullptr, nullptr, a.out, s);
 }
 
 template <Epilogue E>
@@ -463,9 +509,73 @@ bool stream_form(const GemmArgs& a, int splits) {
   return static_cast<int64_t>(a.n / 32) * splits < kFillTiles;
 }
 
+constexpr int kCUs = 256;
+constexpr int kMaxStreamQkv = 288;  // rows of the last form below
+
+// RoPE epilogue, 80 tiles of 16 column pairs: the fewest rows per workgroup that still give each
+// CU at most one (us with weights from HBM, against the partials of pc_gemm_m128 at 2 splits and
+// pc_rope_kv_append_parts: 1 row 5.5 / 6.4, 16 rows 5.8 / 7.0, 37 rows 6.3 / 7.8, 48 rows 6.7 / 8.1,
+// 64 rows 7.7 / 9.2, 96 rows 7.7 / 10.4, 128 rows 8.4 / 10.2, 160 rows 8.9 / 11.6; at 48 rows 32
+// of them per workgroup 7.2, at 64 rows 16 per workgroup 8.9). One 16-row tile alone leaves
+// CUs idle: 160 tiles of 8 pairs (16 rows 5.8, 80 tiles 6.7). Above that 48 rows, two workgroups
+// per CU (256 rows 11.6 / 13.9, the best tile of launch_qkv_rows 12.3).
+int launch_qkv_stream(const QkvArgs& q, hipStream_t s) {
+  const GemmArgs a{q.x, q.w, q.m, kQkvElems, q.k, q.k, 0, 0, nullptr};
+  if (q.m <= 16) return launch_stream<1, 1, 4, 3, kRope>(a, 1, q.positions, q.slots, q.out, s);
+  constexpr int tiles = kQkvElems / 32;
+  constexpr int places = kCUs / tiles;  // X tiles that keep to one workgroup per CU
+  switch ((q.m + 16 * places - 1) / (16 * places)) {
+    case 1: return launch_stream<1, 2, 4, 3, kRope>(a, 1, q.positions, q.slots, q.out, s);
+    case 2: return launch_stream<2, 2, 4, 2, kRope>(a, 1, q.positions, q.slots, q.out, s);
+    case 4: return launch_stream<4, 2, 4, 2, kRope>(a, 1, q.positions, q.slots, q.out, s);
+    default: return launch_stream<3, 2, 4, 2, kRope>(a, 1, q.positions, q.slots, q.out, s);
+  }
+}
+
 }  // namespace
 
 extern "C" {
+
+int pc_qkv_rope_append(void* query_out, void* key_out, void* value_out, const void* x, const void* w, int32_t m, int32_t k,
+                       const int64_t* positions, const void* rope_table, int32_t rope_positions, void* pool,
+                       int64_t num_blocks, int32_t layer, const int64_t* slot_mapping, void* stream) {
+  if (!query_out || !x || !w || !positions || !rope_table) return set_error(PC_ERR_ARGUMENT, "null pointer");
+  if (m < 1 || m > (1 << 16)) return set_error(PC_ERR_ARGUMENT, "m = %d outside [1, 65536]", m);
+  if (k < 64 || k % 64 != 0 || k > kMaxQkvK || static_cast<int64_t>(m) * k > (int64_t{1} << 31)) {
+    return set_error(PC_ERR_ARGUMENT, "k = %d must be a multiple of 64 up to %d, m * k up to 2^31", k, kMaxQkvK);
+  }
+  if (rope_positions < 1) return set_error(PC_ERR_ARGUMENT, "rope_positions must be positive");
+  if ((pool == nullptr) != (slot_mapping == nullptr)) {
+    return set_error(PC_ERR_ARGUMENT, "pool and slot_mapping must both be given or both be null");
+  }
+  if (pool != nullptr) {
+    if (num_blocks < 1 || num_blocks > INT32_MAX) {
+      return set_error(PC_ERR_ARGUMENT, "num_blocks %lld out of range", static_cast<long long>(num_blocks));
+    }
+    if (layer < 0 || layer >= kLayers) return set_error(PC_ERR_ARGUMENT, "layer %d outside [0, 22)", layer);
+  }
+  if (!aligned(query_out, 16) || !aligned(x, 16) || !aligned(w, 16) || !aligned(rope_table, 16) || !aligned(pool, 16) ||
+      !aligned(key_out, 16) || !aligned(value_out, 16)) {
+    return set_error(PC_ERR_ARGUMENT, "buffers must be 16-byte aligned");
+  }
+  QkvArgs a;
+  a.x = static_cast<const _Float16*>(x);
+  a.w = static_cast<const _Float16*>(w);
+  a.m = m;
+  a.k = k;
+  a.positions = positions;
+  a.slots = slot_mapping;
+  a.out.table = static_cast<const _Float16*>(rope_table);
+  a.out.table_positions = rope_positions;
+  a.out.query = static_cast<_Float16*>(query_out);
+  a.out.kind_elems = pool ? num_blocks * kSlots * kRowElems : 0;
+  a.out.layer_pool = pool ? static_cast<_Float16*>(pool) + static_cast<int64_t>(layer) * 2 * a.out.kind_elems : nullptr;
+  a.out.key = static_cast<_Float16*>(key_out);
+  a.out.value = static_cast<_Float16*>(value_out);
+  (void)hipGetLastError();
+  return m <= kMaxStreamQkv ? launch_qkv_stream(a, static_cast<hipStream_t>(stream))
+                       : launch_qkv_rows(a, static_cast<hipStream_t>(stream));
+}
 
 int pc_gemm_m128(void* out, const void* x, const void* w, int32_t m, int32_t n, int32_t k, int32_t splits,
                  int32_t epilogue, void* stream) {

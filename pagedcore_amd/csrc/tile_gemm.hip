@@ -22,6 +22,7 @@
 namespace {
 
 using namespace gemm_device;
+using namespace rope_device;
 using pc_internal::aligned;
 using pc_internal::check_launch;
 using pc_internal::set_error;
@@ -41,13 +42,15 @@ struct TileArgs {
 
 template <int BM, int BN, int WM, int WN, int ST, Epilogue E>
 __global__ __launch_bounds__(64 * WM * WN) void gemm_tile_kernel(const _Float16* x, const _Float16* w, int m, int n,
-                                                                 int k, int ksplit, int ntiles, int mtiles, void* out) {
+                                                                 int k, int ksplit, int ntiles, int mtiles,
+                                                                 const int64_t* positions, const int64_t* slots,
+                                                                 typename OutOf<E>::type out) {
   constexpr int kWaves = WM * WN;
   constexpr int TM = BM / WM, TN = BN / WN, MT = TM / 16, NT = TN / 16;
   constexpr int kXBytes = BM * 128, kStage = (BM + BN) * 128;      // one stage: X rows, then W rows, 128 bytes each
   constexpr int XI = BM / 8 / kWaves, WI = BN / 8 / kWaves;        // DMA instructions per wave and stage
   constexpr int kPer = XI + WI;
-  constexpr int kCols = E == kSwiGLU ? BN / 2 : BN;                // output columns per tile
+  constexpr int kCols = paired(E) ? BN / 2 : BN;                   // output columns (or pairs) per tile
   static_assert(BM % (8 * kWaves) == 0 && BN % (8 * kWaves) == 0 && TN % 32 == 0, "waves share the tile evenly");
   static_assert((ST - 1) * kPer < 64 && ST >= 2 && ST <= 4, "vmcnt counts the later stages");
   extern __shared__ __attribute__((aligned(16))) char smem[];
@@ -69,10 +72,11 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_tile_kernel(const _Float16*
   u -= group * kTileGroup * ntiles;
   const int tile = u / in_group, mtile = kTileGroup * group + u % in_group;
 
-  const int limit = E == kSwiGLU ? n / 2 : n;
+  const int limit = paired(E) ? n / 2 : n;
   // DMA instruction i of a part covers rows 8 i .. 8 i + 7: lane L takes row 8 i + L / 8 and the
   // chunk stored at position L % 8 (chunk c of row r at c ^ (r & 7)). Rows past the matrix
-  // repeat its last row. SwiGLU: each wave's W rows are TN / 2 gate rows, then their up rows.
+  // repeat its last row. SwiGLU: each wave's W rows are TN / 2 gate rows, then their up rows; RoPE:
+  // TN / 2 columns d < 32 of the heads, then their partners d + 32.
   const int row8 = lane >> 3;
   const uint32_t chunk = 16 * ((lane & 7) ^ row8);
   const uint32_t line = 2 * static_cast<uint32_t>(k);
@@ -83,7 +87,11 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_tile_kernel(const _Float16*
   for (int i = 0; i < WI; ++i) {
     const int r = 8 * (i * kWaves + wave) + row8;
     const int last = limit - 1 - kCols * tile;
-    if constexpr (E == kSwiGLU) {
+    if constexpr (E == kRope) {
+      const int base = (r / TN) * (TN / 2), in = r % TN, upper = in >= TN / 2;
+      const int pair = kCols * tile + min(base + in - upper * (TN / 2), last);
+      woff[i] = (pair_row(pair) + upper * kHalfDim) * line + chunk;
+    } else if constexpr (E == kSwiGLU) {
       const int base = (r / TN) * (TN / 2), in = r % TN;
       woff[i] = (in < TN / 2 ? min(base + in, last) : limit + min(base + in - TN / 2, last)) * line + chunk;
     } else {
@@ -92,7 +100,17 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_tile_kernel(const _Float16*
   }
   const int64_t k0 = static_cast<int64_t>(split) * ksplit;
   const char* xbase = reinterpret_cast<const char*>(x + static_cast<int64_t>(BM) * mtile * k + k0);
-  const char* wbase = reinterpret_cast<const char*>(w + static_cast<int64_t>(kCols) * tile * k + k0);
+  const char* wbase = reinterpret_cast<const char*>(w + (E == kRope ? 0 : static_cast<int64_t>(kCols) * tile * k) + k0);
+  // RoPE: the positions and slots of the wave's rows, before the stream (see the end).
+  [[maybe_unused]] int64_t position[MT], token_slot[MT];
+  if constexpr (E == kRope) {
+#pragma unroll
+    for (int j = 0; j < MT; ++j) {
+      const int row = min(BM * mtile + wm * TM + 16 * j + r16, m - 1);
+      position[j] = positions[row];
+      token_slot[j] = (slots != nullptr ? slots : positions)[row];
+    }
+  }
   auto issue = [&](char* stage) {
     asm volatile("" ::: "memory");
 #pragma unroll
@@ -168,11 +186,37 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_tile_kernel(const _Float16*
 
   // acc[i][j] of lane (r16, g), element e: X row wm TM + 16 j + r16, W row wn TN + 16 i + 4 g + e
   // of the tile.
+  [[maybe_unused]] RopeRow rope[MT];
+  [[maybe_unused]] half4_t cs[NT / 2][MT], sn[NT / 2][MT];
+  if constexpr (E == kRope) {  // every table value the wave needs in one round trip
+#pragma unroll
+    for (int j = 0; j < MT; ++j) {
+      rope[j] = rope_row(out, position[j], token_slot[j], slots != nullptr);
+#pragma unroll
+      for (int i = 0; i < NT / 2; ++i) {
+        const _Float16* table = rope[j].table + (kCols * tile + wn * (TN / 2) + 16 * i + 4 * g) % kHalfDim;
+        cs[i][j] = *reinterpret_cast<const half4_t*>(table);
+        sn[i][j] = *reinterpret_cast<const half4_t*>(table + kHalfDim);
+      }
+    }
+  }
 #pragma unroll
   for (int j = 0; j < MT; ++j) {
     const int row = BM * mtile + wm * TM + 16 * j + r16;
     if (row >= m) continue;
-    if constexpr (E == kSwiGLU) {
+    if constexpr (E == kRope) {
+#pragma unroll
+      for (int i = 0; i < NT / 2; ++i) {
+        const int pair = kCols * tile + wn * (TN / 2) + 16 * i + 4 * g;
+        half4_t lo, hi;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          lo[e] = round_h(acc[i][j][e]);
+          hi[e] = round_h(acc[i + NT / 2][j][e]);
+        }
+        if (pair < limit) store_pairs(out, rope[j], row, pair, lo, hi, cs[i][j], sn[i][j]);
+      }
+    } else if constexpr (E == kSwiGLU) {
 #pragma unroll
       for (int i = 0; i < NT / 2; ++i) {
         const int col = kCols * tile + wn * (TN / 2) + 16 * i + 4 * g;
@@ -204,20 +248,25 @@ int64_t tile_count(const TileArgs& a, int bm, int cols, int width) {
 }
 
 template <int BM, int BN, int WM, int WN, int ST, Epilogue E>
-int launch(const TileArgs& a, hipStream_t s) {
+int launch(const TileArgs& a, const int64_t* positions, const int64_t* slots, typename OutOf<E>::type out, hipStream_t s) {
   constexpr int lds = ST * (BM + BN) * 128;
   static_assert(lds <= 160 * 1024, "ring fits the CU's LDS");
   auto kernel = gemm_tile_kernel<BM, BN, WM, WN, ST, E>;
   static std::atomic<uint64_t> raised{0};
   if (int rc = raise_lds_limit(reinterpret_cast<const void*>(kernel), lds, raised)) return rc;
-  constexpr int cols = E == kSwiGLU ? BN / 2 : BN;
-  const int width = E == kSwiGLU ? a.n / 2 : a.n;
+  constexpr int cols = paired(E) ? BN / 2 : BN;
+  const int width = paired(E) ? a.n / 2 : a.n;
   const int ntiles = (width + cols - 1) / cols, mtiles = (a.m + BM - 1) / BM;
   const int64_t total = tile_count(a, BM, cols, width);
   const int64_t grid = (total + kXCDs - 1) / kXCDs * kXCDs;
   hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(grid)), dim3(64 * WM * WN), lds, s, a.x, a.w, a.m, a.n, a.k,
-                     a.ksplit, ntiles, mtiles, a.out);
+                     a.ksplit, ntiles, mtiles, positions, slots, out);
   return check_launch("gemm_tile");
+}
+
+template <int BM, int BN, int WM, int WN, int ST, Epilogue E>
+int launch(const TileArgs& a, hipStream_t s) {
+  return launch<BM, BN, WM, WN, ST, E>(a, nullptr, nullptr, a.out, s);
 }
 
 // The smallest tile of which every CU gets at most one: 64 x 64 (o_proj at 256 rows and 2
@@ -245,6 +294,23 @@ int launch_swiglu(const TileArgs& a, hipStream_t s) {
 }
 
 }  // namespace
+
+namespace gemm_device {
+
+// RoPE epilogue: the smallest tile of which every CU gets at most one, as above, with a stage
+// more where it fits (us, against this file's partials or hipBLASLt and pc_rope_kv_append: 64 x 64
+// at 384 rows 12.5 / 14.5, three stages 14.5; 128 x 64 at 512 rows 17.0 / 18.0, at 768 17.4 / 20.3;
+// 128 x 128 at 1024 rows 25.1 / 26.5, at 1536 25.5 / 28.6). Larger than that it ties: 33.6 / 33.2 at
+// 2048 rows.
+int launch_qkv_rows(const QkvArgs& q, hipStream_t s) {
+  const TileArgs a{q.x, q.w, q.m, kQkvElems, q.k, q.k, nullptr};
+  if (tile_count(a, 64, 64, a.n) <= kCUs) return launch<64, 64, 2, 2, 4, kRope>(a, q.positions, q.slots, q.out, s);
+  if (tile_count(a, 128, 64, a.n) <= kCUs) return launch<128, 64, 4, 2, 4, kRope>(a, q.positions, q.slots, q.out, s);
+  if (tile_count(a, 128, 128, a.n) <= kCUs) return launch<128, 128, 4, 2, 3, kRope>(a, q.positions, q.slots, q.out, s);
+  return launch<128, 192, 4, 2, 3, kRope>(a, q.positions, q.slots, q.out, s);
+}
+
+}  // namespace gemm_device
 
 extern "C" int pc_gemm_rows(void* out, const void* x, const void* w, int32_t m, int32_t n, int32_t k, int32_t splits,
                             int32_t epilogue, void* stream) {

@@ -11,15 +11,15 @@ decode step is one batch-wide pass per layer:
 
   x      = RMSNorm(embedding[ids])                           pc_add_rms_norm
   per layer:
-    qkv  = x @ [Wq; Wk; Wv]^T                                 GEMM: fp32 split-K partials
-    q    = RoPE(q); RoPE(k) and v -> the staged pool slots     pc_rope_kv_append(_parts)
+    q, k, v = x @ [Wq; Wk; Wv]^T; q = RoPE(q);
+      RoPE(k) and v -> the staged pool slots                   one GEMM, pc_qkv_rope_append
     a    = paged attention(q) over the request's blocks        pc_paged_decode_attn
     h   += a @ Wo^T;  x = RMSNorm(h)                           GEMM partials, pc_add_rms_norm(_parts)
     m    = silu(x @ Wgate^T) * (x @ Wup^T)                     one GEMM on [Wgate; Wup], SwiGLU epilogue
     h   += m @ Wdown^T; x = RMSNorm_next(h)                    GEMM partials, pc_add_rms_norm(_parts)
   logits = x @ Wlm^T                                          GEMM (hipBLASLt via torch)
 
-The projections run on pc_gemm_m128 at up to 128 rows (the split-K partial sums are added
+The other projections run on pc_gemm_m128 at up to 128 rows (the split-K partial sums are added
 and rounded to fp16 once by the kernel that consumes them); above that, a prompt's rows among
 them, on pc_gemm_rows or on F.linear (hipBLASLt), whichever is faster at the shape (_rows_splits,
 _rows_swiglu), with pc_silu_mul for the SwiGLU after F.linear. Every elementwise kernel rounds to fp16 where
@@ -241,20 +241,20 @@ def _check_weights(weights: TinyLlamaWeights, what: str) -> None:
         raise ValueError(f"paged {what} requires 22 decoder layers")
 
 
-# Up to GEMM_M128_ROWS rows (a decode step, a short prompt) the q|k|v, o_proj, gate|up and down
-# projections run on pc_gemm_m128: q|k|v, o_proj and down as fp32 split-K partial sums (summed
-# and rounded once by the RoPE / residual-add consumers), gate|up with the SwiGLU epilogue; a
-# 128-token prompt's four take 40 us there, 58 with hipBLASLt and pc_silu_mul. More rows go to
-# pc_gemm_rows where that is faster. Operands the kernels do not take (K not a multiple of
+# Up to GEMM_M128_ROWS rows (a decode step, a short prompt) the o_proj, gate|up and down
+# projections run on pc_gemm_m128: o_proj and down as fp32 split-K partial sums (summed and
+# rounded once by the residual add), gate|up with the SwiGLU epilogue. More rows go to
+# pc_gemm_rows where that is faster. q|k|v, RoPE and the K/V write are one launch at any row count
+# that _qkv_fused takes; eager decode, where the allocator owns the write, projects with one
+# split, which adds in the same order. Operands the kernels do not take (K not a multiple of
 # 64, strided or misaligned weights, ...) use F.linear.
-# Split counts measured on the batch-128 step: q|k|v at 2 (160 workgroups of 32-row tiles,
-# half the partials of 4) 1.930 vs 1.950 ms; o_proj at 2 or 8 and down at 4 or 16 no better.
+# Split counts measured on the batch-128 step: o_proj at 2 or 8 and down at 4 or 16 no better.
 # Up to 64 rows half as many for o_proj and down: the kernel that runs there fills the GPU
 # with them (o_proj 3.4-4.1 us at 2 splits, 3.4-4.4 at 4; down 5.9-8.5 at 4, 6.0-7.8 at 8) and
 # the norm that sums the partials reads half.
 GEMM_M128_ROWS = 128
 GEMM_FEW_ROWS = 64
-QKV_SPLITS = 2
+QKV_SPLITS = 1
 O_PROJ_SPLITS = 4
 DOWN_SPLITS = 8
 
@@ -331,6 +331,23 @@ def _linear_parts(x: Tensor, weight: Tensor, preferred_splits: int) -> Tensor:
     return F.linear(x, weight)
 
 
+def _qkv_fused(rows: int) -> bool:
+    """Whether pc_qkv_rope_append is faster than the projection and the RoPE launch after it: up
+    to one 128 x 128 tile per CU (25.5 / 28.6 us at 1536 rows; 33.6 / 33.2 at 2048)."""
+    return -(-rows // 128) * (QKV_WIDTH // 128) <= 256
+
+
+def _qkv_rope(query: Tensor, x: Tensor, weight: Tensor, positions: Tensor, table: Tensor, **outputs) -> None:
+    """q|k|v = x @ weight.T, RoPE and the K/V write (the outputs of _hip.rope_kv_append): one launch,
+    or the projection and pc_rope_kv_append(_parts)."""
+    if _qkv_fused(x.shape[0]) and weight.shape == (QKV_WIDTH, HIDDEN) and _kernel_operands(x, weight):
+        _hip.qkv_rope_append(query, x, weight, positions, table, **outputs)
+        return
+    qkv = _linear_parts(x, weight, QKV_SPLITS)
+    rope = _hip.rope_kv_append_parts if qkv.ndim == 3 else _hip.rope_kv_append
+    rope(query, qkv, positions, table, **outputs)
+
+
 def _swiglu(x: Tensor, gate_up: Tensor) -> Tensor:
     """fp16(fp16(silu(x @ gate.T)) * fp16(x @ up.T)) for the stacked [gate | up] weight:
     one GEMM launch with the SwiGLU epilogue, or F.linear + pc_silu_mul."""
@@ -359,12 +376,12 @@ def _attention_block(
     x: Tensor, hidden: Tensor, layer: LayerWeights, fused: _FusedLayer, following_norm: Tensor, attend
 ) -> None:
     """One decoder layer around its attention, in place on (x, hidden): q|k|v projection,
-    attend(qkv) -> attention [rows, 2048] (RoPE, KV write and paged attention, supplied by
-    the caller; qkv fp16 [rows, 2560] or fp32 partial sums [splits, rows, 2560]), o_proj +
-    residual + RMSNorm, SwiGLU MLP + residual + the next RMSNorm (reference
+    RoPE, KV write and attention by attend(x, stacked q|k|v weight) -> attention [rows, 2048]
+    (supplied by the caller), o_proj + residual + RMSNorm, SwiGLU MLP + residual + the next
+    RMSNorm (reference
     src/pagedcore/decoder.py:173-193)."""
     fewer = 2 if x.shape[0] <= GEMM_FEW_ROWS else 1
-    attention = attend(_linear_parts(x, fused.qkv, QKV_SPLITS))
+    attention = attend(x, fused.qkv)
     _add_rms_norm(x, hidden, _linear_parts(attention, layer.o_proj, O_PROJ_SPLITS // fewer), layer.post_attention_norm)
     activated = _swiglu(x, fused.gate_up)
     _add_rms_norm(x, hidden, _linear_parts(activated, layer.down_proj, DOWN_SPLITS // fewer), following_norm)
@@ -410,7 +427,8 @@ def decode_paged(
         workspaces: Dict[int, Tensor] = {}
         for index, layer in enumerate(weights.layers):
 
-            def attend(qkv: Tensor, index: int = index) -> Tensor:
+            def attend(x: Tensor, weight: Tensor, index: int = index) -> Tensor:
+                qkv = _linear_parts(x, weight, QKV_SPLITS)
                 query = allocator.write_decode_layers_rotary(request_ids, index, qkv, table)
                 out, workspace = attend_rows(query, allocator, request_ids, index)
                 workspaces[workspace.data_ptr()] = workspace
@@ -551,11 +569,8 @@ class DecodeGraph:
         attention = torch.empty_like(query)
         for index, layer in enumerate(weights.layers):
 
-            def attend(qkv: Tensor, index: int = index) -> Tensor:
-                if qkv.ndim == 3:
-                    _hip.rope_kv_append_parts(query, qkv, positions, self._table, pool=pool, layer=index, slot_mapping=slots)
-                else:
-                    _hip.rope_kv_append(query, qkv, positions, self._table, pool=pool, layer=index, slot_mapping=slots)
+            def attend(x: Tensor, weight: Tensor, index: int = index) -> Tensor:
+                _qkv_rope(query, x, weight, positions, self._table, pool=pool, layer=index, slot_mapping=slots)
                 _hip.planned_decode_attention(attention, query, pool, index, self._lens, self._plan, MAX_BLOCKS, self._workspace)
                 return attention.view(batch, HIDDEN)
 
@@ -688,7 +703,7 @@ def prefill_paged(
     """Prefill one admitted, empty request from int64 [1, T] prompt ids; returns fp16
     logits [1, T, vocab]. Only K is rotated (reference src/pagedcore/decoder.py:113-135).
 
-    The K/V write is fused into the forward: per layer, pc_rope_kv_append rotates Q and K
+    The K/V write is fused into the forward: per layer, RoPE and the append rotate Q and K
     and writes the rotated K and the V straight into the slots the append takes (staged
     through KVAllocator.append_prompt), besides the contiguous copy the prompt's attention
     reads. The append is published only after the whole forward succeeded, as the
@@ -730,9 +745,8 @@ def _prefill_forward(ids: Tensor, positions: Tensor, slots: Tensor, weights: Tin
     attended = torch.empty_like(query)
     for index, layer in enumerate(weights.layers):
 
-        def attend(qkv: Tensor, index: int = index) -> Tensor:
-            rope = _hip.rope_kv_append_parts if qkv.ndim == 3 else _hip.rope_kv_append
-            rope(query, qkv, positions, table, key_out=key, value_out=value, pool=pool, layer=index, slot_mapping=slots)
+        def attend(x: Tensor, weight: Tensor, index: int = index) -> Tensor:
+            _qkv_rope(query, x, weight, positions, table, key_out=key, value_out=value, pool=pool, layer=index, slot_mapping=slots)
             if on_layer is not None:
                 on_layer(index)
             _hip.prefill_attention(attended, query, key, value)

@@ -131,6 +131,31 @@ def test_fused_decode_write_checks_before_any_write():
     assert allocator.capacity() == counts
 
 
+@pytest.mark.parametrize("rows", [1, 129, 1536, 1537])
+@pytest.mark.parametrize("form", ["plain", "strided", "misaligned"])
+def test_qkv_route_takes_only_what_the_kernel_reads(monkeypatch, rows, form):
+    """_qkv_rope gives pc_qkv_rope_append contiguous, aligned weights up to 1536 rows and every
+    other call to the projection and a RoPE launch, with the same outputs passed on."""
+    n, k = dec.QKV_WIDTH, dec.HIDDEN
+    x = torch.zeros((rows, k), dtype=torch.float16)
+    if form == "strided":
+        weight = torch.zeros((n, 2 * k), dtype=torch.float16)[:, ::2]
+    elif form == "misaligned":
+        weight = torch.zeros(n * k + 1, dtype=torch.float16)[1:].view(n, k)
+    else:
+        weight = torch.zeros((n, k), dtype=torch.float16)
+    calls = []
+    monkeypatch.setattr(_hip, "qkv_rope_append", lambda q, x, w, p, t, **out: calls.append(("fused", out)))
+    monkeypatch.setattr(_hip, "rope_kv_append", lambda q, qkv, p, t, **out: calls.append(("rope", out)))
+    monkeypatch.setattr(_hip, "rope_kv_append_parts", lambda q, qkv, p, t, **out: calls.append(("parts", out)))
+    monkeypatch.setattr(_hip, "gemm_m128", lambda out, x, w, **options: None)
+    monkeypatch.setattr(torch.nn.functional, "linear", lambda x, w: torch.zeros((x.shape[0], w.shape[0]), dtype=torch.float16))
+    outputs = {"pool": x, "layer": 2, "slot_mapping": x}
+    dec._qkv_rope(x, x, weight, None, None, **outputs)
+    expected = "fused" if form == "plain" and rows <= 1536 else "rope"
+    assert [name for name, _ in calls] == [expected] and calls[0][1] == outputs
+
+
 @pytest.mark.parametrize("rows", [1, 64, 128, 129, 384, 640, 1024, 2048])
 @pytest.mark.parametrize("form", ["plain", "strided", "misaligned", "odd_k", "odd_n"])
 def test_projection_route_takes_only_what_the_kernels_read(monkeypatch, rows, form):

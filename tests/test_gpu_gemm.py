@@ -356,3 +356,90 @@ def test_rope_kv_append_instances(device, splits, outputs):
             assert torch.equal(pool[21, 1].view(-1, 4, 64)[slots[kept]], values[kept])
     for a, b in zip(*results):
         assert np.array_equal(_bits(a), _bits(b))
+
+
+# --- pc_qkv_rope_append (the q|k|v projection with RoPE and the KV write as its epilogue) ------
+
+
+def _qkv_inputs(device, m, k, seed):
+    gen = torch.Generator(device=device).manual_seed(seed)
+    x = torch.randn((m, k), device=device, generator=gen).half()
+    w = (0.05 * torch.randn((2560, k), device=device, generator=gen)).half()
+    positions = torch.randint(0, 2048, (m,), device=device, generator=gen)
+    blocks = m // 16 + 2
+    slots = torch.randperm(blocks * 16, device=device, generator=gen)[:m].contiguous()
+    return x, w, positions, slots, blocks
+
+
+# The edges of the forms' rows: 16 rows; then 48 per X tile of 16, up to 192; 288; and one workgroup
+# per CU of 64 x 64, 128 x 64 and 128 x 128 tiles.
+@pytest.mark.parametrize("m", [1, 7, 16, 17, 48, 49, 96, 97, 144, 145, 192, 193, 288, 289, 384, 385, 768, 769, 1536, 1537])
+@pytest.mark.parametrize("k", [64, 320, 2048])
+def test_qkv_rope_append_forms(device, m, k):
+    """Every output against float64: the projection within its fp32 accumulation (k 2^-24 of the
+    sum of magnitudes) and one rounding, the rotation within its three; pool rows equal to the
+    contiguous ones; rows of tokens without a slot, and memory past the outputs, untouched."""
+    x, w, positions, slots, blocks = _qkv_inputs(device, m, k, 7 * m + k)
+    dropped = torch.arange(m, device=device) % 5 == 3
+    slots[dropped] = torch.where(torch.arange(m, device=device)[dropped] % 2 == 0, -1, blocks * 16)
+    table = dec.rope_table(device)
+    pool = torch.full((22, 2, blocks, 16, 4, 64), 7.0, dtype=torch.float16, device=device)
+    guard = torch.full((3, m * 2048 + 64), 7.0, dtype=torch.float16, device=device)
+    query = guard[0, : m * 2048].view(m, 32, 64)
+    key, value = (guard[i, : m * 256].view(m, 4, 64) for i in (1, 2))
+    _hip.qkv_rope_append(query, x, w, positions, table, key_out=key, value_out=value, pool=pool, layer=3, slot_mapping=slots)
+    torch.cuda.synchronize()
+    assert (guard[0, m * 2048 :] == 7.0).all() and (guard[1:, m * 256 :] == 7.0).all()
+    flat = pool[3].view(2, -1, 4, 64)
+    kept = slots[~dropped]
+    assert torch.equal(flat[0][kept], key[~dropped]) and torch.equal(flat[1][kept], value[~dropped])
+    untouched = torch.ones(blocks * 16, dtype=torch.bool, device=device)
+    untouched[kept] = False
+    assert (flat[:, untouched] == 7.0).all() and (pool[:3] == 7.0).all() and (pool[4:] == 7.0).all()
+
+    y = x.double() @ w.double().T
+    delta = k * 2.0**-24 * (x.double().abs() @ w.double().abs().T)
+    delta = delta + 2.0**-11 * (y.abs() + delta) + 2.0**-25  # one rounding to fp16
+    heads, errors = y.view(m, 40, 64), delta.view(m, 40, 64)
+    c, s = (table[positions, i].double()[:, None] for i in (0, 1))
+    lo, hi = heads[:, :36, :32], heads[:, :36, 32:]
+    elo, ehi = errors[:, :36, :32], errors[:, :36, 32:]
+    got = torch.cat((query, key), 1).double()
+    for part, a, b, ea, eb, sign in ((got[..., :32], lo, hi, elo, ehi, -1), (got[..., 32:], hi, lo, ehi, elo, 1)):
+        exact = a * c + sign * b * s
+        moved = ea * c.abs() + eb * s.abs()
+        magnitudes = (a * c).abs() + (b * s).abs() + moved
+        bound = moved + 2.0**-11 * 2 * magnitudes * (1 + 2.0**-10) + 3 * 2.0**-25
+        assert ((part - exact).abs() <= bound).all()
+    assert ((value.double() - heads[:, 36:]).abs() <= errors[:, 36:]).all()
+
+
+@pytest.mark.parametrize("m", [1, 16, 17, 48, 49, 64])
+def test_qkv_rope_append_adds_as_the_projection_with_one_split(device, m):
+    """The same bits as pc_gemm_m128 with one split and pc_rope_kv_append_parts, which eager decode
+    runs; each output left out in turn; a position past the table gives NaN rows (v kept) and
+    no pool write."""
+    x, w, positions, slots, blocks = _qkv_inputs(device, m, 2048, m)
+    positions[m // 2] = 2048
+    table = dec.rope_table(device)
+    parts = torch.empty((1, m, 2560), dtype=torch.float32, device=device)
+    _hip.gemm_m128(parts, x, w)
+    for outputs in ("pool", "contiguous", "both"):
+        results = []
+        for fused in (False, True):
+            pool = torch.full((22, 2, blocks, 16, 4, 64), 7.0, dtype=torch.float16, device=device)
+            query = torch.empty(m, 32, 64, dtype=torch.float16, device=device)
+            key = torch.full((m, 4, 64), 7.0, dtype=torch.float16, device=device)
+            value = torch.full_like(key, 7.0)
+            given = {} if outputs == "pool" else {"key_out": key, "value_out": value}
+            if outputs != "contiguous":
+                given.update(pool=pool, layer=0, slot_mapping=slots)
+            if fused:
+                _hip.qkv_rope_append(query, x, w, positions, table, **given)
+            else:
+                _hip.rope_kv_append_parts(query, parts, positions, table, **given)
+            torch.cuda.synchronize()
+            assert query[m // 2].isnan().all()
+            results.append((query, key, value, pool))
+        for a, b in zip(*results):
+            assert np.array_equal(_bits(a), _bits(b))

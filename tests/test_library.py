@@ -304,6 +304,36 @@ def test_gemm_rejects_invalid_arguments_without_a_gpu(overrides, needle):
     assert needle in lib.pc_last_error()
 
 
+@pytest.mark.parametrize(
+    "overrides,needle",
+    [
+        ({"query": None}, b"null pointer"),
+        ({"w": None}, b"null pointer"),
+        ({"m": 0}, b"m = 0"),
+        ({"m": 65537}, b"65536"),
+        ({"k": 96}, b"multiple of 64"),
+        ({"k": 0}, b"multiple of 64"),
+        ({"k": (1 << 18) + 64}, b"multiple of 64"),
+        ({"m": 65536, "k": 65536}, b"2^31"),
+        ({"rope": 0}, b"rope_positions"),
+        ({"slots": None}, b"both"),
+        ({"blocks": 0}, b"num_blocks"),
+        ({"layer": 22}, b"layer 22"),
+        ({"x": 264}, b"aligned"),
+        ({"key": 264}, b"aligned"),
+    ],
+)
+def test_qkv_rope_append_rejects_invalid_arguments_without_a_gpu(overrides, needle):
+    lib = _hip.load()
+    a = {"query": 256, "key": 256, "x": 256, "w": 256, "m": 4, "k": 2048, "rope": 2048, "pool": 256, "blocks": 4,
+         "layer": 0, "slots": 256}
+    a.update(overrides)
+    status = lib.pc_qkv_rope_append(a["query"], a["key"], a["key"], a["x"], a["w"], a["m"], a["k"], 256, 256, a["rope"],
+                                    a["pool"], a["blocks"], a["layer"], a["slots"], None)
+    assert status == 1
+    assert needle in lib.pc_last_error()
+
+
 def test_split_k_consumers_reject_invalid_arguments_without_a_gpu():
     lib = _hip.load()
     assert lib.pc_add_rms_norm_parts(256, 256, None, 1, 256, 4, 2048, 1e-5, None) == 1
