@@ -88,6 +88,10 @@ struct QkvArgs {
   rope_device::RopeOut out;
 };
 int launch_qkv_rows(const QkvArgs& a, hipStream_t s);  // the tiles of a prompt's rows
+// SwiGLU at most of a decode step's rows on those tiles: where they are faster, and the launch
+// (k a multiple of 64, n of 64).
+bool swiglu_short_tiles(int m, int n, int k);
+int launch_swiglu_short(void* out, const _Float16* x, const _Float16* w, int m, int n, int k, hipStream_t s);
 
 }  // namespace gemm_device
 

@@ -639,6 +639,7 @@ int pc_gemm_m128(void* out, const void* x, const void* w, int32_t m, int32_t n, 
         if (m <= 48) return launch_stream<3, 3, 4, 2, kSwiGLU>(a, splits, s);
         return launch_stream<4, 3, 4, 2, kSwiGLU>(a, splits, s);
       }
+      if (k % 64 == 0 && swiglu_short_tiles(m, n, k)) return launch_swiglu_short(out, a.x, a.w, m, n, k, s);
       a.half_rows = n / 2;
       a.tiles = n / (2 * kSwiGLUHalf);
       return launch<64, 64, 4, 8, kSwiGLU>(a, splits, s);

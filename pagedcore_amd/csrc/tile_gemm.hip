@@ -281,13 +281,13 @@ int launch_plain(const TileArgs& a, hipStream_t s) {
   return launch<128, 192, 4, 2, 3, E>(a, s);
 }
 
-// SwiGLU (no splits): the same rule over 128-row tiles of 64, 96 and 128 output columns (gate|up
-// at 256 rows 23.3 us against 31.0 for hipBLASLt and pc_silu_mul, at 512 rows 30.8 / 37.5, at 640
-// rows 37.4 / 40.9); where none fits one round, 96 columns with two stages, two workgroups per
-// CU (1024 rows 50.9 / 58.0, 2048 rows 95.6 / 101.7).
+// SwiGLU (no splits): the same rule over 128-row tiles of 48, 96 and 128 output columns (gate|up
+// at 256 rows 22.6 us against 31.0 for hipBLASLt and pc_silu_mul, at 160 rows 20.8 (64 columns,
+// eight waves: 23.1); at 512 rows 30.8 / 37.5, at 640 rows 37.4 / 40.9); where none fits one round,
+// 96 columns with two stages, two workgroups per CU (1024 rows 50.9 / 58.0, 2048 rows 95.6 / 101.7).
 int launch_swiglu(const TileArgs& a, hipStream_t s) {
   const int width = a.n / 2;
-  if (tile_count(a, 128, 64, width) <= kCUs) return launch<128, 128, 4, 2, 3, kSwiGLU>(a, s);
+  if (tile_count(a, 128, 48, width) <= kCUs) return launch<128, 96, 4, 1, 3, kSwiGLU>(a, s);
   if (tile_count(a, 128, 96, width) <= kCUs) return launch<128, 192, 4, 2, 3, kSwiGLU>(a, s);
   if (tile_count(a, 128, 128, width) <= kCUs) return launch<128, 256, 2, 4, 3, kSwiGLU>(a, s);
   return launch<128, 192, 4, 2, 2, kSwiGLU>(a, s);
@@ -308,6 +308,17 @@ int launch_qkv_rows(const QkvArgs& q, hipStream_t s) {
   if (tile_count(a, 128, 64, a.n) <= kCUs) return launch<128, 64, 4, 2, 4, kRope>(a, q.positions, q.slots, q.out, s);
   if (tile_count(a, 128, 128, a.n) <= kCUs) return launch<128, 128, 4, 2, 3, kRope>(a, q.positions, q.slots, q.out, s);
   return launch<128, 192, 4, 2, 3, kRope>(a, q.positions, q.slots, q.out, s);
+}
+
+// 64 x 96 tiles (48 output columns) for 81 to 128 rows, one workgroup per CU: gate|up moves 655 KB
+// into each of 236 CUs, where gemm_m128_kernel moves 768 KB into each of 176 (128 rows 16.5 us /
+// 17.7, 96 rows 15.5 / 16.4, 80 rows 15.9 / 15.7; five to seven stages 17.0 to 17.8).
+bool swiglu_short_tiles(int m, int n, int k) {
+  return m > 80 && m <= 128 && k <= kMaxK && 2 * ((n / 2 + 47) / 48) <= kCUs;
+}
+
+int launch_swiglu_short(void* out, const _Float16* x, const _Float16* w, int m, int n, int k, hipStream_t s) {
+  return launch<64, 96, 4, 1, 4, kSwiGLU>(TileArgs{x, w, m, n, k, k, out}, s);
 }
 
 }  // namespace gemm_device

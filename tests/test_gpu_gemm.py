@@ -105,6 +105,25 @@ def test_gemm_swiglu_equals_silu_mul_of_the_fp16_projections(device, m):
     assert ((fused.float() - expected).abs() <= 2 * ulp + 2.0**-24).all()
 
 
+@pytest.mark.parametrize("m", [80, 81, 127, 128])
+@pytest.mark.parametrize("n,k", [(64, 64), (192, 192), (320, 2048), (11264, 256), (12352, 128)])
+def test_gemm_swiglu_short_tiles(device, m, n, k):
+    """Either side of the rows and columns that take 64 x 96 tiles, columns that end inside a tile,
+    fewer K stages than the ring has: bit equal to pc_silu_mul of the fp16 projections, and
+    nothing written past the output."""
+    x, w = _inputs(device, m, n, k, seed=3 * m + n + k)
+    guard = torch.full((m * (n // 2) + 64,), -77.0, dtype=torch.float16, device=device)
+    fused = guard[: m * (n // 2)].view(m, n // 2).fill_(float("nan"))
+    _hip.gemm_m128(fused, x, w, epilogue=_hip.GEMM_SWIGLU)
+    projected = torch.empty((m, n), dtype=torch.float16, device=device)
+    _hip.gemm_m128(projected, x, w, epilogue=_hip.GEMM_HALF)
+    separate = torch.empty((m, n // 2), dtype=torch.float16, device=device)
+    _hip.silu_mul(separate, projected)
+    torch.cuda.synchronize()
+    assert (guard[m * (n // 2) :] == -77.0).all()
+    assert np.array_equal(_bits(fused), _bits(separate))
+
+
 def _sum_in_split_order(parts: torch.Tensor) -> torch.Tensor:
     total = parts[0].clone()
     for s in range(1, parts.shape[0]):
@@ -243,7 +262,7 @@ def test_gemm_row_and_tile_edges(device, m, n, k, splits):
 # --- pc_gemm_rows (a prompt's rows) -----------------------------------------------------------
 
 # (n, k, splits, rows): every tile shape of the dispatch (64 x 64, 64 x 128, 128 x 128,
-# 128 x 192; SwiGLU 64, 96 and 128 output columns, and 96 on two stages), rows one short of, at
+# 128 x 192; SwiGLU 48, 96 and 128 output columns, and 96 on two stages), rows one short of, at
 # and one past a tile, column counts that end inside a tile, fewer K stages than the ring has.
 ROWS_SHAPES = [
     (64, 64, 1, (1, 63, 64, 65, 200)),
