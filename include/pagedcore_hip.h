@@ -166,6 +166,17 @@ int pc_paged_decode_attn_noalloc(void* out, const void* query, const void* pool,
                                  int32_t num_records, void* stream);
 
 /*
+ * The fault word of `workspace` once everything enqueued on `stream` before this call is done,
+ * without a synchronization of the stream: a kernel writes it, with the caller's `ticket`,
+ * into `host`, 8 bytes of pinned (device-visible, coherent) memory, which this call polls for up
+ * to 200 us. Returns the word (>= 0), -pc_status, or PC_ATTN_FAULTS_PENDING if it did not
+ * arrive in that time (the caller then synchronizes and reads the workspace itself). `host` must
+ * not be in use by another call, and `ticket` must differ from the last one used with it.
+ */
+#define PC_ATTN_FAULTS_PENDING -16
+int64_t pc_attn_read_faults(const void* workspace, void* host, uint32_t ticket, void* stream);
+
+/*
  * Host-side decode plan (no device access). context_lens [batch] and block_tables
  * [batch][max_blocks] are HOST arrays (row b: sequence b's physical blocks in logical order,
  * only the first ceil(len / 16) read); plan is HOST memory of `capacity` rows of

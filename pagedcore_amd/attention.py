@@ -9,8 +9,8 @@ replaced by one launch of the HIP paged-attention kernels, which walk the block 
 the device; nothing larger than the output is materialised from the pool.
 
 Both entry points fail closed on a device-side failure of the launch (a cut sequence's
-merge that timed out or saw another XCD's flag, a block id outside the pool): they read
-the workspace's fault word after the launch, which synchronizes, and raise
+merge that timed out or saw another XCD's flag, a block id outside the pool): they wait
+for the launch, read the workspace's fault word and raise
 AttentionFaultError (a RuntimeError) instead of returning NaN rows.
 
 ``paged_attention_batch`` is the batched form the decode loop needs (one launch for all
@@ -47,19 +47,17 @@ def attend_rows(
     """One launch of paged attention for already validated rows; returns the output and
     the workspace whose fault word the caller must check (check_attention_faults) before
     it trusts the output. Nothing synchronizes."""
-    tables, lengths = allocator.gather_block_tables(request_ids, layer_index=layer_index)
+    rows = allocator.decode_rows(request_ids, layer_index=layer_index)
     pool = allocator.pool
     if pool.device != query.device:
         raise ValueError("query and KV cache must be on the same device")
     if not query.is_cuda:
         raise RuntimeError("paged attention runs on the GPU: the KV pool and query must be on a CUDA device")
     batch = len(request_ids)
-    q = query.reshape(batch, Q_HEADS, HEAD_DIM)
-    if not q.is_contiguous():
-        q = q.contiguous()
+    q = query if query.is_contiguous() else query.contiguous()
     out = torch.empty((batch, Q_HEADS, 1, HEAD_DIM), dtype=torch.float16, device=query.device)
-    plan = allocator.decode_plan(request_ids, layer_index=layer_index)
-    workspace = _hip.paged_decode_attention(out, q, pool, layer_index, tables, lengths, plan=plan)
+    plan = allocator.rows_plan(rows)
+    workspace = _hip.paged_decode_attention(out, q, pool, layer_index, rows.tables, rows.lengths, plan=plan)
     return out, workspace
 
 

@@ -759,7 +759,15 @@ class KVAllocator:
         """Device decode plan (pc_attn_plan rows: balanced bins of the batch's blocks) for the
         batch that gather_block_tables returns, built once per allocator state from the host
         tables, so the 22 layers of a decode step share it."""
-        batch = self._gather(request_ids, layer_index)
+        return self.rows_plan(self._gather(request_ids, layer_index))
+
+    def decode_rows(self, request_ids: Sequence[RequestId], *, layer_index: int) -> _DecodeBatch:
+        """gather_block_tables (its checks and tables) for a caller that also takes the plan of
+        the same rows: rows_plan(decode_rows(...)) checks the allocator's state once."""
+        return self._gather(request_ids, layer_index)
+
+    def rows_plan(self, batch: _DecodeBatch) -> Tensor:
+        """decode_plan of the rows that decode_rows returned."""
         if batch.plan is None:
             plan = _hip.decode_plan(batch.host_lengths, batch.host_tables)
             batch.plan = _upload(plan, self._pool.device)

@@ -910,3 +910,49 @@ def test_stale_raised_flags_are_not_taken(device, stale):
     # the slots the plan uses were consumed and lowered; the others keep their planted flags
     used = check_decode_plan(plan, w.lengths, w.tables, w.num_blocks, nbytes)["slots"]
     assert int((workspace_flags(planted) == 0).sum().item()) == used * 4
+
+
+# --- reading the fault word (polled, or by a synchronizing copy) --------------------------------
+
+
+def test_fault_word_is_read_after_the_streams_work(device):
+    """The polled word is the one that the work enqueued before the read leaves, call after call;
+    behind work far longer than the poll (several ms of products) the copy reads it."""
+    workspace = torch.zeros(256, dtype=torch.uint8, device=device)
+    word = _hip.fault_word(workspace)
+    for value in (0, 1, 4, 0, 7, 2, 0):
+        word.fill_(value)
+        assert _hip._read_fault_word(workspace) == value
+    big = torch.randn((8192, 8192), device=device).half()
+    for value in (3, 0):
+        for _ in range(8):
+            big @ big
+        word.fill_(value)
+        assert _hip._read_fault_word(workspace) == value
+
+
+def test_fault_words_of_threads_and_streams_do_not_mix(device):
+    """Each of four threads, alternating between two streams of its own, reads back the words
+    it wrote."""
+    import threading
+
+    failures = []
+
+    def work(index):
+        streams = [torch.cuda.Stream(device) for _ in range(2)]
+        spaces = [torch.zeros(256, dtype=torch.uint8, device=device) for _ in range(2)]
+        torch.cuda.synchronize()
+        for turn in range(50):
+            with torch.cuda.stream(streams[turn % 2]):
+                value = (turn * 4 + index) % 8
+                _hip.fault_word(spaces[turn % 2]).fill_(value)
+                got = _hip._read_fault_word(spaces[turn % 2])
+                if got != value:
+                    failures.append((index, turn, value, got))
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(4)]
+    for thread in threads:
+        thread.start()
+    for thread in threads:
+        thread.join()
+    assert not failures

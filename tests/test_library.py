@@ -334,6 +334,13 @@ def test_qkv_rope_append_rejects_invalid_arguments_without_a_gpu(overrides, need
     assert needle in lib.pc_last_error()
 
 
+@pytest.mark.parametrize("workspace,host,needle", [(None, 8, b"null"), (256, None, b"null"), (128, 8, b"aligned"), (256, 4, b"aligned")])
+def test_read_faults_rejects_invalid_arguments_without_a_gpu(workspace, host, needle):
+    lib = _hip.load()
+    assert lib.pc_attn_read_faults(workspace, host, 1, None) == -1
+    assert needle in lib.pc_last_error()
+
+
 def test_split_k_consumers_reject_invalid_arguments_without_a_gpu():
     lib = _hip.load()
     assert lib.pc_add_rms_norm_parts(256, 256, None, 1, 256, 4, 2048, 1e-5, None) == 1
