@@ -28,7 +28,7 @@
 // per layer, against eight waves per workgroup without these (same outputs bit for bit for
 // KG = 1): 64 tokens 3.8 -> 3.1, 333 7.3 -> 5.7, 512 9.0 -> 6.9, 1024 14.8 -> 10.6, 2048 31.1 ->
 // 26.5. Slower: three stages (28.7 at 2048, 6.7 at 333), 32 queries per wave (34.2), packed
-// fp16 conversion (29.8 against 28.6), K prefetched across steps.
+// fp16 conversion (29.8 against 28.6).
 
 #include <hip/hip_runtime.h>
 
