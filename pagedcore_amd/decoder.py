@@ -484,7 +484,7 @@ def capture_graph(fn: Callable[[], T], device: torch.device) -> Tuple[torch.cuda
 class DecodeGraph:
     """decode_paged for batches of up to a fixed size, captured once as a HIP graph and replayed.
 
-    A decode step is about 200 launches (9 per layer); issued one by one from Python they
+    A decode step is about 155 launches (7 per layer); issued one by one from Python they
     cost more host time than the GPU needs to run them. Here the step's device work is
     captured once, with every per-step input in static device buffers: token ids, the
     staged token's slot and position of each row, the staged context lengths, and the
@@ -762,8 +762,8 @@ class PrefillGraph:
     and replayed, returning only the logits of the prompt's last position (what greedy
     generation selects from).
 
-    prefill_paged issues about 200 launches from Python (about 2.6 ms of host time at any
-    prompt length), so short prompts are host-bound. Here the forward is captured at
+    prefill_paged issues about 160 launches from Python (the same host time at any prompt
+    length), so short prompts are host-bound. Here the forward is captured at
     `tokens` rows over static inputs: token ids, slot mapping and the index of the last
     real row (positions are 0 .. tokens - 1: the cache is empty). A shorter prompt is
     padded at the end; causal attention keeps every real row blind to the padding rows
