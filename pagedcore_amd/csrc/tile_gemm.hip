@@ -269,14 +269,16 @@ int launch(const TileArgs& a, hipStream_t s) {
   return launch<BM, BN, WM, WN, ST, E>(a, nullptr, nullptr, a.out, s);
 }
 
-// The smallest tile of which every CU gets at most one: 64 x 64 (o_proj at 256 rows and 2
-// splits 7.1 us, hipBLASLt 9.4), 64 x 128 (o_proj at 512 rows 9.2 / 11.2), 128 x 128 (down at
-// 512 rows and 4 splits 19.1 / 28.0, at 1024 and 2 splits 31.3 / 40.0), 128 x 192 (down at 640
-// rows and 4 splits 24.2 / 32.8). A second round of workgroups costs more than larger tiles.
+// The smallest tile of which every CU gets at most one, with a fourth stage where it fits (us with
+// weights from HBM and the norm that consumes the output, against three stages): 64 x 64 (o_proj at
+// 256 rows and 2 splits 11.3 / 12.3, at 512 rows unsplit 15.5), 128 x 64 (down at
+// 160 rows and 4 splits 16.2 / 16.4, at 256 rows 17.7 / 18.1; 64 x 128 17.3 and 19.0), 128 x 128 (down
+// at 512 rows and 4 splits 25.2, four stages 25.1), 128 x 192 (down at 640 rows
+// and 4 splits 29.5). A second round of workgroups costs more than larger tiles.
 template <Epilogue E>
 int launch_plain(const TileArgs& a, hipStream_t s) {
-  if (tile_count(a, 64, 64, a.n) <= kCUs) return launch<64, 64, 2, 2, 3, E>(a, s);
-  if (tile_count(a, 64, 128, a.n) <= kCUs) return launch<64, 128, 2, 4, 3, E>(a, s);
+  if (tile_count(a, 64, 64, a.n) <= kCUs) return launch<64, 64, 2, 2, 4, E>(a, s);
+  if (tile_count(a, 128, 64, a.n) <= kCUs) return launch<128, 64, 4, 2, 4, E>(a, s);
   if (tile_count(a, 128, 128, a.n) <= kCUs) return launch<128, 128, 4, 2, 3, E>(a, s);
   return launch<128, 192, 4, 2, 3, E>(a, s);
 }

@@ -263,16 +263,16 @@ def _rows_splits(rows: int, n: int, k: int) -> int:
     """K splits for pc_gemm_rows above GEMM_M128_ROWS rows, or 0 where F.linear (hipBLASLt) is
     the faster product. By the count of 128 x 128 tiles against the 256 CUs: few tiles want K
     split (a long K more), and pay for it in partials that the consumer reads; about one per
-    two CUs still win unsplit; more are the library's. Measured, us here / library (the
-    consumer reads the partials in 1-3 us): o_proj 7.1 / 9.4 at 256 rows and 9.2 / 11.2 at 512
-    (2 splits), 13.8 / 15.6 at 1024 (unsplit), 22.1 / 22.1 at 2048; q|k|v 9.2 / 10.7 at 384 (2),
-    13.6 / 15.0 at 768 (unsplit), 12.8 / 13.2 at 512, 28.0 / 27.8 at 2048; down 14.5 / 20.6 at
-    256, 19.1 / 28.0 at 512, 24.2 / 32.8 at 640 (4), 31.3 / 40.0 at 1024 (2), 30.0 / 32.4 at 768
-    (2), 56.8 / 55.8 at 2048."""
+    two to four CUs win unsplit; more are the library's. Measured, us of the product alone, here /
+    library: o_proj 7.1 / 9.4 at 256 rows and 9.2 / 11.2 at 512 (2 splits), 13.8 / 15.6 at 1024
+    (unsplit), 22.1 / 22.1 at 2048; down 14.5 / 20.6 at 256, 19.1 / 28.0 at 512, 24.2 / 32.8 at 640
+    (4), 31.3 / 40.0 at 1024 (2), 56.8 / 55.8 at 2048. With weights from HBM and the norm that
+    consumes the output: o_proj at 512 rows 15.5 unsplit, 16.1 at 2 splits; 19.0 / 18.4 at 640; down
+    34.6 / 36.3 at 768 (2)."""
     tiles = -(-rows // 128) * -(-n // 128)
     if k >= 4096:
-        return 4 if tiles <= 80 else 2 if 100 < tiles <= 128 else 0
-    return 2 if tiles <= 64 else 1 if 100 <= tiles <= 128 else 0
+        return 4 if tiles <= 80 else 2 if tiles <= 128 else 0
+    return 2 if tiles <= 48 else 1 if tiles <= 64 or 100 <= tiles <= 128 else 0
 
 
 def _rows_swiglu(rows: int, width: int) -> bool:

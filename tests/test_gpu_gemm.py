@@ -261,7 +261,7 @@ def test_gemm_row_and_tile_edges(device, m, n, k, splits):
 
 # --- pc_gemm_rows (a prompt's rows) -----------------------------------------------------------
 
-# (n, k, splits, rows): every tile shape of the dispatch (64 x 64, 64 x 128, 128 x 128,
+# (n, k, splits, rows): every tile shape of the dispatch (64 x 64, 128 x 64, 128 x 128,
 # 128 x 192; SwiGLU 48, 96 and 128 output columns, and 96 on two stages), rows one short of, at
 # and one past a tile, column counts that end inside a tile, fewer K stages than the ring has.
 ROWS_SHAPES = [
