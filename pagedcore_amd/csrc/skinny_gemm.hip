@@ -479,6 +479,16 @@ int launch_stream(const GemmArgs& a, int splits, hipStream_t s) {
   return launch_stream<MT, NT, WAVES, D, E>(a, splits, nullptr, nullptr, a.out, s);
 }
 
+constexpr int kCUs = 256;
+
+// X tile (in 16 rows) of a launch with `wtiles` W tiles: the fewest rows per workgroup that give each
+// CU at most one workgroup, up to 64; beyond that 48 rows, of which two workgroups fit a CU.
+int x_tile(int m, int wtiles) {
+  const int places = wtiles < kCUs ? kCUs / wtiles : 1;
+  const int mt = (m + 16 * places - 1) / (16 * places);
+  return mt <= 4 ? mt : 3;
+}
+
 template <Epilogue E>
 int launch_stream_rows(const GemmArgs& a, int mt, int splits, hipStream_t s) {
   switch (mt) {
@@ -509,7 +519,6 @@ bool stream_form(const GemmArgs& a, int splits) {
   return static_cast<int64_t>(a.n / 32) * splits < kFillTiles;
 }
 
-constexpr int kCUs = 256;
 constexpr int kMaxStreamQkv = 288;  // rows of the last form below
 
 // RoPE epilogue, 80 tiles of 16 column pairs: the fewest rows per workgroup that still give each
@@ -522,9 +531,7 @@ constexpr int kMaxStreamQkv = 288;  // rows of the last form below
 int launch_qkv_stream(const QkvArgs& q, hipStream_t s) {
   const GemmArgs a{q.x, q.w, q.m, kQkvElems, q.k, q.k, 0, 0, nullptr};
   if (q.m <= 16) return launch_stream<1, 1, 4, 3, kRope>(a, 1, q.positions, q.slots, q.out, s);
-  constexpr int tiles = kQkvElems / 32;
-  constexpr int places = kCUs / tiles;  // X tiles that keep to one workgroup per CU
-  switch ((q.m + 16 * places - 1) / (16 * places)) {
+  switch (x_tile(q.m, kQkvElems / 32)) {
     case 1: return launch_stream<1, 2, 4, 3, kRope>(a, 1, q.positions, q.slots, q.out, s);
     case 2: return launch_stream<2, 2, 4, 2, kRope>(a, 1, q.positions, q.slots, q.out, s);
     case 4: return launch_stream<4, 2, 4, 2, kRope>(a, 1, q.positions, q.slots, q.out, s);
@@ -533,6 +540,31 @@ int launch_qkv_stream(const QkvArgs& q, hipStream_t s) {
 }
 
 }  // namespace
+
+namespace gemm_device {
+
+// The rows and columns of the q|k|v projection above, so that an unsplit product of 2560 columns has
+// pc_qkv_rope_append's bits at every row count (from 289 rows both are on tiles, which all add in one
+// order). It and narrower products are also faster here than on 64 x 64 tiles (us: n 2560 at 160
+// rows 6.9 / 10.5, at 288 9.5 / 10.6; n 2048 at 256 rows 7.0 / 10.4; n 512 4.9 / 10.3), wider ones
+// hardly or not (n 5632 at 160 rows 14.6 / 14.9, at 96 12.2 / 11.5).
+bool rows_stream(int m, int n) { return m <= kMaxStreamQkv && n <= kQkvElems; }
+
+int launch_rows_stream(void* out, const _Float16* x, const _Float16* w, int m, int n, int k, Epilogue epilogue,
+                       hipStream_t s) {
+  const GemmArgs a{x, w, m, n, k, k, 0, 0, out};
+  const int mt = x_tile(m, n / 32);
+  if (epilogue == kHalf) return launch_stream_rows<kHalf>(a, mt, 1, s);
+  if (epilogue == kPartials) return launch_stream_rows<kPartials>(a, mt, 1, s);
+  switch (mt) {
+    case 1: return launch_stream<1, 1, 4, 3, kSwiGLU>(a, 1, s);
+    case 2: return launch_stream<2, 3, 4, 2, kSwiGLU>(a, 1, s);
+    case 3: return launch_stream<3, 3, 4, 2, kSwiGLU>(a, 1, s);
+    default: return launch_stream<4, 3, 4, 2, kSwiGLU>(a, 1, s);
+  }
+}
+
+}  // namespace gemm_device
 
 extern "C" {
 

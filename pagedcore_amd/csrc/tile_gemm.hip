@@ -351,6 +351,7 @@ extern "C" int pc_gemm_rows(void* out, const void* x, const void* w, int32_t m, 
     return set_error(PC_ERR_ARGUMENT, "n = %d must be a multiple of %d", n, epilogue == kSwiGLU ? 64 : 32);
   }
   (void)hipGetLastError();
+  if (splits == 1 && rows_stream(m, n)) return launch_rows_stream(out, a.x, a.w, m, n, k, static_cast<Epilogue>(epilogue), s);
   if (epilogue == kSwiGLU) return launch_swiglu(a, s);
   return epilogue == kHalf ? launch_plain<kHalf>(a, s) : launch_plain<kPartials>(a, s);
 }

@@ -246,8 +246,8 @@ def _check_weights(weights: TinyLlamaWeights, what: str) -> None:
 # rounded once by the residual add), gate|up with the SwiGLU epilogue. More rows go to
 # pc_gemm_rows where that is faster. q|k|v, RoPE and the K/V write are one launch at any row count
 # that _qkv_fused takes; eager decode, where the allocator owns the write, projects with one
-# split, which adds in the same order. Operands the kernels do not take (K not a multiple of
-# 64, strided or misaligned weights, ...) use F.linear.
+# split, which adds in the same order (_qkv_projection). Operands the kernels do not take (K not a
+# multiple of 64, strided or misaligned weights, ...) use F.linear.
 # Split counts measured on the batch-128 step: o_proj at 2 or 8 and down at 4 or 16 no better.
 # Up to 64 rows half as many for o_proj and down: the kernel that runs there fills the GPU
 # with them (o_proj 3.4-4.1 us at 2 splits, 3.4-4.4 at 4; down 5.9-8.5 at 4, 6.0-7.8 at 8) and
@@ -337,10 +337,28 @@ def _qkv_fused(rows: int) -> bool:
     return -(-rows // 128) * (QKV_WIDTH // 128) <= 256
 
 
+def _qkv_in_one_launch(x: Tensor, weight: Tensor) -> bool:
+    """Whether _qkv_rope is the one launch of pc_qkv_rope_append."""
+    return _qkv_fused(x.shape[0]) and weight.shape == (QKV_WIDTH, HIDDEN) and _kernel_operands(x, weight)
+
+
+def _qkv_projection(x: Tensor, weight: Tensor) -> Tensor:
+    """q|k|v = x @ weight.T for a caller that rotates and writes it itself: the values that _qkv_rope
+    rotates, bit for bit (so decode_paged and a DecodeGraph agree), as fp32 partial sums of one
+    split or the fp16 product. pc_gemm_m128 and pc_gemm_rows add an unsplit product of 2560
+    columns in pc_qkv_rope_append's order."""
+    rows = x.shape[0]
+    if rows <= GEMM_M128_ROWS or not _qkv_in_one_launch(x, weight):
+        return _linear_parts(x, weight, QKV_SPLITS)
+    qkv = torch.empty((rows, QKV_WIDTH), dtype=torch.float16, device=x.device)
+    _hip.gemm_rows(qkv, x, weight, epilogue=_hip.GEMM_HALF)
+    return qkv
+
+
 def _qkv_rope(query: Tensor, x: Tensor, weight: Tensor, positions: Tensor, table: Tensor, **outputs) -> None:
     """q|k|v = x @ weight.T, RoPE and the K/V write (the outputs of _hip.rope_kv_append): one launch,
     or the projection and pc_rope_kv_append(_parts)."""
-    if _qkv_fused(x.shape[0]) and weight.shape == (QKV_WIDTH, HIDDEN) and _kernel_operands(x, weight):
+    if _qkv_in_one_launch(x, weight):
         _hip.qkv_rope_append(query, x, weight, positions, table, **outputs)
         return
     qkv = _linear_parts(x, weight, QKV_SPLITS)
@@ -428,7 +446,7 @@ def decode_paged(
         for index, layer in enumerate(weights.layers):
 
             def attend(x: Tensor, weight: Tensor, index: int = index) -> Tensor:
-                qkv = _linear_parts(x, weight, QKV_SPLITS)
+                qkv = _qkv_projection(x, weight)
                 query = allocator.write_decode_layers_rotary(request_ids, index, qkv, table)
                 out, workspace = attend_rows(query, allocator, request_ids, index)
                 workspaces[workspace.data_ptr()] = workspace
@@ -505,7 +523,7 @@ class DecodeGraph:
 
     Same checks, errors and staged-append semantics as decode_paged for any 1 to `batch`
     requests (any requests, in any order, step to step). A batch of exactly `batch`
-    requests runs the kernels decode_paged runs, at the same shapes, so its logits and
+    requests adds every product in the order decode_paged does, so its logits and
     cache bytes equal decode_paged's. A smaller batch is padded to `batch` rows: a padding
     row has no slot (it writes nothing to the pool) and context length 0 (no attention
     work, its output row is never written), and its logits are dropped. The GEMMs then run

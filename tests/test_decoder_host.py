@@ -156,6 +156,32 @@ def test_qkv_route_takes_only_what_the_kernel_reads(monkeypatch, rows, form):
     assert [name for name, _ in calls] == [expected] and calls[0][1] == outputs
 
 
+@pytest.mark.parametrize("rows,route", [(1, "m128"), (128, "m128"), (129, "rows"), (1536, "rows"), (1537, "library")])
+@pytest.mark.parametrize("form", ["plain", "strided", "misaligned"])
+def test_eager_qkv_route_adds_as_the_fused_launch(monkeypatch, rows, route, form):
+    """_qkv_projection takes the kernels that add in pc_qkv_rope_append's order, unsplit, wherever
+    _qkv_rope takes that launch, and F.linear wherever it does not."""
+    n, k = dec.QKV_WIDTH, dec.HIDDEN
+    x = torch.zeros((rows, k), dtype=torch.float16)
+    if form == "strided":
+        weight = torch.zeros((n, 2 * k), dtype=torch.float16)[:, ::2]
+    elif form == "misaligned":
+        weight = torch.zeros(n * k + 1, dtype=torch.float16)[1:].view(n, k)
+    else:
+        weight = torch.zeros((n, k), dtype=torch.float16)
+    calls = []
+
+    def product(name):
+        return lambda out, x, w, *, splits=1, epilogue=_hip.GEMM_PARTIALS: calls.append((name, splits, out.shape[-2:]))
+
+    monkeypatch.setattr(_hip, "gemm_m128", product("m128"))
+    monkeypatch.setattr(_hip, "gemm_rows", product("rows"))
+    monkeypatch.setattr(torch.nn.functional, "linear", lambda x, w: torch.zeros((x.shape[0], w.shape[0]), dtype=torch.float16))
+    qkv = dec._qkv_projection(x, weight)
+    assert qkv.shape[-2:] == (rows, n) and qkv.ndim == (3 if calls and route == "m128" else 2)
+    assert calls == ([(route, 1, (rows, n))] if form == "plain" and route != "library" else [])
+
+
 @pytest.mark.parametrize("rows", [1, 64, 128, 129, 384, 640, 1024, 2048])
 @pytest.mark.parametrize("form", ["plain", "strided", "misaligned", "odd_k", "odd_n"])
 def test_projection_route_takes_only_what_the_kernels_read(monkeypatch, rows, form):

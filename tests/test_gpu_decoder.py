@@ -434,6 +434,31 @@ def test_decode_graph_replays_equal_decode_paged(device):
         torch.randn(1000, device=device).sum().item()  # unrelated eager work between replays
 
 
+@pytest.mark.parametrize("batch", [129, 257, 300])
+def test_decode_graph_equals_decode_paged_above_128_rows(device, batch):
+    """At the row counts where q|k|v leaves pc_gemm_m128: logits and pool bytes of a DecodeGraph of
+    exactly `batch` rows equal eager decode_paged's, bit for bit, over two steps."""
+    weights = _synthetic(device)
+    requests = tuple(RequestId(str(row)) for row in range(batch))
+    pools = [torch.zeros((22, 2, 2 * batch, 16, 4, 64), dtype=torch.float16, device=device) for _ in range(2)]
+    eager, graphed = (KVAllocator(pool) for pool in pools)
+    for allocator in (eager, graphed):
+        gen = torch.Generator(device=device).manual_seed(batch)
+        for row, request in enumerate(requests):
+            allocator.create(KVReservation(request, 2))
+            length = 1 + row % 20
+            cached = torch.randn((2, 22, length, 4, 64), device=device, generator=gen).half()
+            allocator.append(request, cached[0], cached[1])
+    graph = dec.DecodeGraph(weights, graphed, batch=batch)
+    for step in range(2):
+        tokens = torch.tensor([[(5 * step + row) % 31] for row in range(batch)], device=device)
+        expected = dec.decode_paged(tokens, weights, eager, requests)
+        got = graph.step(tokens, requests)
+        torch.cuda.synchronize()
+        assert torch.equal(got, expected)
+        assert torch.equal(pools[0].view(torch.int16), pools[1].view(torch.int16))
+
+
 def test_decode_graph_pads_smaller_batches(device):
     """A DecodeGraph of 6 rows stepping 1, 4, 6 and 3 requests against eager decode_paged on
     a twin pool: the padding rows write nothing (every pool byte outside the real rows'

@@ -462,3 +462,26 @@ def test_qkv_rope_append_adds_as_the_projection_with_one_split(device, m):
             results.append((query, key, value, pool))
         for a, b in zip(*results):
             assert np.array_equal(_bits(a), _bits(b))
+
+
+# Either side of the row tiles of the stream form up to 288 rows, then of the tile forms, then the library.
+@pytest.mark.parametrize("m", [65, 97, 128, 129, 144, 145, 192, 193, 256, 257, 288, 289, 384, 385, 600, 768, 769, 1536, 1537])
+def test_eager_projection_has_the_bits_of_the_fused_launch(device, m):
+    """The q|k|v projection of eager decode, rotated and written by the RoPE launch, against
+    pc_qkv_rope_append (what a DecodeGraph issues): the same bits at every row count."""
+    x, w, positions, slots, blocks = _qkv_inputs(device, m, 2048, m)
+    table = dec.rope_table(device)
+    results = []
+    for fused in (False, True):
+        pool = torch.full((22, 2, blocks, 16, 4, 64), 7.0, dtype=torch.float16, device=device)
+        query = torch.empty(m, 32, 64, dtype=torch.float16, device=device)
+        outputs = {"pool": pool, "layer": 1, "slot_mapping": slots}
+        if fused:
+            dec._qkv_rope(query, x, w, positions, table, **outputs)
+        else:
+            qkv = dec._qkv_projection(x, w)
+            (_hip.rope_kv_append_parts if qkv.ndim == 3 else _hip.rope_kv_append)(query, qkv, positions, table, **outputs)
+        torch.cuda.synchronize()
+        results.append((query, pool))
+    for a, b in zip(*results):
+        assert torch.equal(a.view(torch.int16), b.view(torch.int16))
