@@ -309,7 +309,8 @@ int pc_gemm_m128(void* out, const void* x, const void* w, int32_t m, int32_t n, 
  *
  * Replaces torch.nn.functional.linear on a prompt's activations (reference
  * src/pagedcore/dense.py:91-104, called per layer by src/pagedcore/decoder.py:113-135). An unsplit
- * product of 2560 columns is added in the order of pc_qkv_rope_append's, as pc_gemm_m128's is.
+ * product of 2560 columns (k from 256) is added in the order of pc_qkv_rope_append's, as
+ * pc_gemm_m128's is.
  */
 int pc_gemm_rows(void* out, const void* x, const void* w, int32_t m, int32_t n, int32_t k, int32_t splits,
                  int32_t epilogue, void* stream);

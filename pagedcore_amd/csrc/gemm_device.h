@@ -94,7 +94,7 @@ bool swiglu_short_tiles(int m, int n, int k);
 int launch_swiglu_short(void* out, const _Float16* x, const _Float16* w, int m, int n, int k, hipStream_t s);
 // An unsplit product of a prompt's rows on the streams of a decode step: where, and the launch (k a
 // multiple of 64, n of 32, for SwiGLU of 64).
-bool rows_stream(int m, int n);
+bool rows_stream(int m, int n, int k);
 int launch_rows_stream(void* out, const _Float16* x, const _Float16* w, int m, int n, int k, Epilogue epilogue, hipStream_t s);
 
 }  // namespace gemm_device

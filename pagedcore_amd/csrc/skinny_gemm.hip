@@ -489,34 +489,74 @@ int x_tile(int m, int wtiles) {
   return mt <= 4 ? mt : 3;
 }
 
+// A form of gemm_stream_kernel: 16 mt rows of X times 16 nt rows of W per workgroup.
+struct StreamTile {
+  int mt, nt;
+};
+constexpr StreamTile kStreamTiles[] = {{1, 2}, {2, 2}, {3, 2}, {4, 2}, {2, 3}, {3, 3}, {4, 3}};
+
 template <Epilogue E>
-int launch_stream_rows(const GemmArgs& a, int mt, int splits, hipStream_t s) {
-  switch (mt) {
+int launch_stream_tile(const GemmArgs& a, StreamTile t, int splits, hipStream_t s) {
+  switch (t.mt + (t.nt == 3 ? 10 : 0)) {
     case 1: return launch_stream<1, 2, 4, 2, E>(a, splits, s);
     case 2: return launch_stream<2, 2, 4, 2, E>(a, splits, s);
     case 3: return launch_stream<3, 2, 4, 2, E>(a, splits, s);
-    default: return launch_stream<4, 2, 4, 2, E>(a, splits, s);
+    case 4: return launch_stream<4, 2, 4, 2, E>(a, splits, s);
+    case 12: return launch_stream<2, 3, 4, 2, E>(a, splits, s);
+    case 13: return launch_stream<3, 3, 4, 2, E>(a, splits, s);
+    default: return launch_stream<4, 3, 4, 2, E>(a, splits, s);
   }
 }
 
-constexpr int kFillTiles = 224;  // 32-row W tiles (times splits) that keep 256 CUs busy
+int64_t rounds(int64_t workgroups) { return (workgroups + kCUs - 1) / kCUs; }
 
-// Whether a call runs on gemm_stream_kernel: by m, n, k and splits alone, not by epilogue, and
-// always with four waves, so that one product has the same bits under every epilogue and
-// for every m up to 64. Measured with weights streaming from HBM (us, stream against
-// gemm_m128_kernel, whose time hardly depends on m):
-//   up to 32 rows: always (gate|up 9.9-11.5 / 14.5-15.2, q|k|v at 2 splits 3.6-4.1 / 6.1-6.4,
-//     o_proj at 4 splits 3.3-3.7 / 4.2-4.4, down at 4 splits 5.8-6.8 / 8.3-8.6);
-//   up to 64 rows: unless split-K gives the 64-row tiles of gemm_m128_kernel a workgroup for
-//     most CUs (down at 8 splits: 7.7 / 7.5 at 48 rows, 8.6 / 7.8 at 64); else 13.9 / 14.9 for
-//     gate|up at 64 rows, 4.4 / 4.6 for o_proj, 5.1 / 6.5 for q|k|v;
-//   above: only where 32-row W tiles leave CUs idle (q|k|v at 2 splits, 128 rows: 6.3 / 6.9;
-//     gate|up 20.5 / 17.6).
-bool stream_form(const GemmArgs& a, int splits) {
-  if (a.ksplit % 64 != 0 || a.k > (1 << 24)) return false;  // row offsets in 32 bits
-  if (a.m <= 32) return true;
-  if (a.m <= 64) return !(splits > 1 && a.n % 64 == 0 && (a.n / 64) * splits >= 176);
-  return static_cast<int64_t>(a.n / 32) * splits < kFillTiles;
+// 64-row W tiles of gemm_m128_kernel: with eight waves when they alone fill the GPU's workgroup
+// slots; with four waves (2 x 4 register tiles per wave) when they give 160 to 175 workgroups,
+// where 32-row tiles would need more workgroups than one round on the CUs (q|k|v at 4
+// splits: 7.5 vs 8.3 us); else 32-row tiles with four waves.
+enum M128Tile { k32x4, k64x4, k64x8 };
+M128Tile m128_tile(int n, int splits) {
+  const int64_t tiles64 = n % 64 == 0 ? static_cast<int64_t>(n / 64) * splits : 0;
+  if (tiles64 >= 176) return k64x8;
+  return tiles64 >= 160 && static_cast<int64_t>(n / 32) * splits > kCUs ? k64x4 : k32x4;
+}
+
+// Which form takes a call, from an estimate of its time (us; a constant common to all is left out):
+// rounds of workgroups on the CUs times a round's setup and the bytes it moves into a CU. A later
+// round overlaps an earlier one where workgroups share a CU (two of up to 80 KB of LDS; three of 48 KB,
+// while a K range is short enough for the L2 to hold what they share). The constants are fitted to
+// the times of every form at 22800 calls (m 1 to 128, n 32 to 37000, k 64 to 16000, 1 to 16
+// splits, weights from HBM): the form taken is 2 % off the fastest on average; it is more than 5 %
+// slower than gemm_m128_kernel alone at 0.4 % of them (17 % at most) and 36 % faster on average. A
+// rule on the number of W tiles was more than 5 % slower at 11 % of them, by up to 56 % (SwiGLU of n 14336
+// at 64 rows 20.7 / 15.0, 299 tiles of 48 rows; n 7136, k 256 at 111 rows 5.8 / 4.1).
+float stream_time(const GemmArgs& a, int splits, StreamTile t) {
+  const int64_t workgroups =
+      static_cast<int64_t>((a.n + 16 * t.nt - 1) / (16 * t.nt)) * splits * ((a.m + 16 * t.mt - 1) / (16 * t.mt));
+  const int lds_kb = 16 * (t.mt + t.nt), units = a.ksplit / 64;
+  const int64_t r = rounds(workgroups);
+  const float overlap = r == 1 || lds_kb > 80 ? 1.0f : lds_kb > 48 || units > 16 ? 0.88f : 0.75f;
+  const float round = (lds_kb > 80 ? 0.7f : 0.22f) + 0.074f * (t.mt + t.nt) * ((units + 3) / 4);  // units per wave
+  return overlap * r * round + 0.066e-6f * a.n * static_cast<float>(a.k);
+}
+
+float m128_time(const GemmArgs& a, int splits, M128Tile t) {
+  const int nt = t == k32x4 ? 2 : 4;
+  const int64_t r = rounds(static_cast<int64_t>(a.n / (16 * nt)) * splits);
+  const float overlap = r == 1 || t != k32x4 ? 1.0f : 0.8f;
+  return 0.15f + overlap * r * (0.055f + 0.022f * (8 + nt) * (a.ksplit / 64));
+}
+
+// The fastest stream form, of those with 48-row W tiles alone if `wide`, and its time.
+StreamTile stream_tile(const GemmArgs& a, int splits, bool wide, float& time) {
+  StreamTile best{1, 2};
+  time = INFINITY;
+  for (const StreamTile t : kStreamTiles) {
+    if (16 * (t.mt - 1) >= a.m || (wide && t.nt != 3)) continue;
+    const float estimate = stream_time(a, splits, t);
+    if (estimate < time) time = estimate, best = t;
+  }
+  return best;
 }
 
 constexpr int kMaxStreamQkv = 288;  // rows of the last form below
@@ -545,17 +585,17 @@ namespace gemm_device {
 
 // The rows and columns of the q|k|v projection above, so that an unsplit product of 2560 columns has
 // pc_qkv_rope_append's bits at every row count (from 289 rows both are on tiles, which all add in one
-// order). It and narrower products are also faster here than on 64 x 64 tiles (us: n 2560 at 160
+// order; k from 256, where every wave has a unit). It and narrower products are also faster here than on 64 x 64 tiles (us: n 2560 at 160
 // rows 6.9 / 10.5, at 288 9.5 / 10.6; n 2048 at 256 rows 7.0 / 10.4; n 512 4.9 / 10.3), wider ones
 // hardly or not (n 5632 at 160 rows 14.6 / 14.9, at 96 12.2 / 11.5).
-bool rows_stream(int m, int n) { return m <= kMaxStreamQkv && n <= kQkvElems; }
+bool rows_stream(int m, int n, int k) { return m <= kMaxStreamQkv && n <= kQkvElems && k >= 256; }
 
 int launch_rows_stream(void* out, const _Float16* x, const _Float16* w, int m, int n, int k, Epilogue epilogue,
                        hipStream_t s) {
   const GemmArgs a{x, w, m, n, k, k, 0, 0, out};
   const int mt = x_tile(m, n / 32);
-  if (epilogue == kHalf) return launch_stream_rows<kHalf>(a, mt, 1, s);
-  if (epilogue == kPartials) return launch_stream_rows<kPartials>(a, mt, 1, s);
+  if (epilogue == kHalf) return launch_stream_tile<kHalf>(a, {mt, 2}, 1, s);
+  if (epilogue == kPartials) return launch_stream_tile<kPartials>(a, {mt, 2}, 1, s);
   switch (mt) {
     case 1: return launch_stream<1, 1, 4, 3, kSwiGLU>(a, 1, s);
     case 2: return launch_stream<2, 3, 4, 2, kSwiGLU>(a, 1, s);
@@ -565,6 +605,33 @@ int launch_rows_stream(void* out, const _Float16* x, const _Float16* w, int m, i
 }
 
 }  // namespace gemm_device
+
+namespace {
+
+// Whether a call of pc_gemm_m128 runs on gemm_stream_kernel: by m, n, k and splits alone, not by
+// epilogue (an unsplit product only if every epilogue gains), and always with four waves, so that one
+// product has the same bits under every epilogue, and under two row counts that are sent to
+// the same kernel (each projection of the decoder from 1 to 64 rows, and from 65 to 128).
+constexpr float kMargin = 1.1f;  // where the estimates are close, gemm_m128_kernel
+bool stream_form(const GemmArgs& a, int splits) {
+  if (a.ksplit % 64 != 0 || a.k > (1 << 24)) return false;  // row offsets in 32 bits
+  if (splits == 1 && rows_stream(a.m, a.n, a.k)) return true;
+  // A K range of fewer units than waves leaves waves idle (n 1024, k 128 per split, 48 rows: 3.5
+  // us / 3.1; k 64, n 15488, SwiGLU at 12 rows 4.2 / 3.2).
+  const int units = a.ksplit / 64;
+  if (units < 4 && a.m > 16 * units) return false;
+  if (units == 1 && splits == 1 && a.n > 48 * kCUs) return false;
+  if (a.m <= 16) return true;
+  float time;
+  if (splits == 1 && a.n % 64 == 0) {  // SwiGLU, which has tiles of its own
+    stream_tile(a, 1, true, time);
+    if (kMargin * time >= m128_time(a, 1, k64x8)) return false;
+  }
+  stream_tile(a, splits, false, time);
+  return kMargin * time < m128_time(a, splits, m128_tile(a.n, splits));
+}
+
+}  // namespace
 
 extern "C" {
 
@@ -637,39 +704,37 @@ int pc_gemm_m128(void* out, const void* x, const void* w, int32_t m, int32_t n, 
     case kHalf:
       if (epilogue == kHalf && splits != 1) return set_error(PC_ERR_ARGUMENT, "fp16 output needs one split");
       if (n % 32 != 0) return set_error(PC_ERR_ARGUMENT, "n = %d must be a multiple of 32", n);
+      if (splits == 1 && rows_stream(m, n, k)) return launch_rows_stream(out, a.x, a.w, m, n, k, static_cast<Epilogue>(epilogue), s);
       if (stream_form(a, splits)) {
-        // X tiles of up to 64 rows when the W tiles fill the CUs; else smaller ones, so that
-        // several workgroups share a W tile (q|k|v at 2 splits, 160 W tiles, 48 rows: 4.5 us
-        // on 3 x 160 workgroups of 16 rows, 4.8 on 160 of 48).
-        const int rows16 = (m + 15) / 16;
-        const bool fills = static_cast<int64_t>(n / 32) * splits >= kFillTiles;
-        const int mt = rows16 <= 2 ? rows16 : fills ? (rows16 < 4 ? rows16 : 4) : rows16 == 3 ? 1 : rows16 == 4 ? 2 : 3;
-        return epilogue == kHalf ? launch_stream_rows<kHalf>(a, mt, splits, s) : launch_stream_rows<kPartials>(a, mt, splits, s);
+        float time;
+        const StreamTile t = stream_tile(a, splits, false, time);
+        return epilogue == kHalf ? launch_stream_tile<kHalf>(a, t, splits, s) : launch_stream_tile<kPartials>(a, t, splits, s);
       }
-      // 64-row tiles with eight waves when they alone fill the GPU's workgroup slots; with
-      // four waves (2 x 4 register tiles per wave) when they give 160 to 175 workgroups, where
-      // 32-row tiles would need more workgroups than one round on the CUs (q|k|v at 4
-      // splits: 7.5 vs 8.3 us); else 32-row tiles with four waves.
-      if (n % 64 == 0 && (n / 64) * splits >= 176) {
-        a.tiles = n / 64;
-        return epilogue == kHalf ? launch<64, 64, 4, 8, kHalf>(a, splits, s) : launch<64, 64, 4, 8, kPartials>(a, splits, s);
+      switch (m128_tile(n, splits)) {
+        case k64x8:
+          a.tiles = n / 64;
+          return epilogue == kHalf ? launch<64, 64, 4, 8, kHalf>(a, splits, s) : launch<64, 64, 4, 8, kPartials>(a, splits, s);
+        case k64x4:
+          a.tiles = n / 64;
+          return epilogue == kHalf ? launch<64, 64, 4, 4, kHalf>(a, splits, s) : launch<64, 64, 4, 4, kPartials>(a, splits, s);
+        default:
+          a.tiles = n / 32;
+          return epilogue == kHalf ? launch<32, 64, 4, 4, kHalf>(a, splits, s) : launch<32, 64, 4, 4, kPartials>(a, splits, s);
       }
-      if (n % 64 == 0 && (n / 64) * splits >= 160 && (n / 32) * splits > 256) {
-        a.tiles = n / 64;
-        return epilogue == kHalf ? launch<64, 64, 4, 4, kHalf>(a, splits, s) : launch<64, 64, 4, 4, kPartials>(a, splits, s);
-      }
-      a.tiles = n / 32;
-      return epilogue == kHalf ? launch<32, 64, 4, 4, kHalf>(a, splits, s) : launch<32, 64, 4, 4, kPartials>(a, splits, s);
     case kSwiGLU:
       if (splits != 1) return set_error(PC_ERR_ARGUMENT, "the SwiGLU epilogue needs one split");
       if (n % (2 * kSwiGLUHalf) != 0) return set_error(PC_ERR_ARGUMENT, "n = %d must be a multiple of 64", n);
+      if (rows_stream(m, n, k)) return launch_rows_stream(out, a.x, a.w, m, n, k, kSwiGLU, s);
       // One tile per 8 NT gate rows: 704 small tiles at one X tile (11.0 us at 16 rows, 235
       // tiles of 24 gate rows the same), 235 above it (14.6 -> 11.5 us at 32 rows).
       if (stream_form(a, splits)) {
         if (m <= 16) return launch_stream<1, 1, 4, 3, kSwiGLU>(a, splits, s);
-        if (m <= 32) return launch_stream<2, 3, 4, 2, kSwiGLU>(a, splits, s);
-        if (m <= 48) return launch_stream<3, 3, 4, 2, kSwiGLU>(a, splits, s);
-        return launch_stream<4, 3, 4, 2, kSwiGLU>(a, splits, s);
+        float time;
+        switch (stream_tile(a, splits, true, time).mt) {
+          case 2: return launch_stream<2, 3, 4, 2, kSwiGLU>(a, splits, s);
+          case 3: return launch_stream<3, 3, 4, 2, kSwiGLU>(a, splits, s);
+          default: return launch_stream<4, 3, 4, 2, kSwiGLU>(a, splits, s);
+        }
       }
       if (k % 64 == 0 && swiglu_short_tiles(m, n, k)) return launch_swiglu_short(out, a.x, a.w, m, n, k, s);
       a.half_rows = n / 2;

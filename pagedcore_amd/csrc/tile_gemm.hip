@@ -314,9 +314,10 @@ int launch_qkv_rows(const QkvArgs& q, hipStream_t s) {
 
 // 64 x 96 tiles (48 output columns) for 81 to 128 rows, one workgroup per CU: gate|up moves 655 KB
 // into each of 236 CUs, where gemm_m128_kernel moves 768 KB into each of 176 (128 rows 16.5 us /
-// 17.7, 96 rows 15.5 / 16.4, 80 rows 15.9 / 15.7; five to seven stages 17.0 to 17.8).
+// 17.7, 96 rows 15.5 / 16.4, 80 rows 15.9 / 15.7; five to seven stages 17.0 to 17.8). A short K does not
+// repay the setup (at k 64 and 128 8 to 12 % slower, from 1024 level, from 2048 2 % faster and more).
 bool swiglu_short_tiles(int m, int n, int k) {
-  return m > 80 && m <= 128 && k <= kMaxK && 2 * ((n / 2 + 47) / 48) <= kCUs;
+  return m > 80 && m <= 128 && k >= 1024 && k <= kMaxK && 2 * ((n / 2 + 47) / 48) <= kCUs;
 }
 
 int launch_swiglu_short(void* out, const _Float16* x, const _Float16* w, int m, int n, int k, hipStream_t s) {
@@ -351,7 +352,7 @@ extern "C" int pc_gemm_rows(void* out, const void* x, const void* w, int32_t m, 
     return set_error(PC_ERR_ARGUMENT, "n = %d must be a multiple of %d", n, epilogue == kSwiGLU ? 64 : 32);
   }
   (void)hipGetLastError();
-  if (splits == 1 && rows_stream(m, n)) return launch_rows_stream(out, a.x, a.w, m, n, k, static_cast<Epilogue>(epilogue), s);
+  if (splits == 1 && rows_stream(m, n, k)) return launch_rows_stream(out, a.x, a.w, m, n, k, static_cast<Epilogue>(epilogue), s);
   if (epilogue == kSwiGLU) return launch_swiglu(a, s);
   return epilogue == kHalf ? launch_plain<kHalf>(a, s) : launch_plain<kPartials>(a, s);
 }

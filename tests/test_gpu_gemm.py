@@ -259,6 +259,67 @@ def test_gemm_row_and_tile_edges(device, m, n, k, splits):
         assert np.array_equal(_bits(fused), _bits(separate))
 
 
+# (n, k, splits): K ranges of one to three units (fewer than waves); short splits in several rounds; 48-row W
+# tiles of every epilogue that end inside a tile, at one and at two rounds; columns where
+# 64-row tiles of all rows take one round and 48-row tiles do not.
+FORM_SHAPES = [(64, 64, 1), (96, 192, 1), (1024, 1024, 8), (512, 512, 8), (4096, 512, 8), (11296, 256, 1), (20480, 320, 1), (14336, 256, 1), (3104, 1536, 4)]
+
+
+@pytest.mark.parametrize("m", [16, 17, 32, 33, 40, 48, 49, 64, 65, 96, 97, 128])
+@pytest.mark.parametrize("n,k,splits", FORM_SHAPES)
+def test_gemm_forms(device, m, n, k, splits):
+    """Shapes on either side of the choice between the kernel's forms: partials against float64 split
+    by split, nothing written past the output, and with one split the same sums under every
+    epilogue."""
+    x, w = _inputs(device, m, n, k, seed=7 * m + n + k)
+    guard = torch.full((splits * m * n + 64,), -77.0, dtype=torch.float32, device=device)
+    out = guard[: splits * m * n].view(splits, m, n).fill_(float("nan"))
+    _hip.gemm_m128(out, x, w, splits=splits, epilogue=_hip.GEMM_PARTIALS)
+    torch.cuda.synchronize()
+    assert (guard[splits * m * n :] == -77.0).all()
+    span = k // splits
+    for s in range(splits):
+        xs, ws = x[:, s * span : (s + 1) * span].double(), w[:, s * span : (s + 1) * span].double()
+        bound = span * 2.0**-24 * (xs.abs() @ ws.abs().t())  # `span` exact products added in fp32, in any order
+        assert ((out[s].double() - xs @ ws.t()).abs() <= bound).all()
+    if splits == 1:
+        half = torch.empty((m, n), dtype=torch.float16, device=device)
+        _hip.gemm_m128(half, x, w, epilogue=_hip.GEMM_HALF)
+        assert np.array_equal(_bits(half), _bits(out[0].half()))
+        if n % 64 == 0:
+            fused = torch.full((m * (n // 2) + 64,), -77.0, dtype=torch.float16, device=device)
+            _hip.gemm_m128(fused[: m * (n // 2)].view(m, n // 2), x, w, epilogue=_hip.GEMM_SWIGLU)
+            separate = torch.empty((m, n // 2), dtype=torch.float16, device=device)
+            _hip.silu_mul(separate, half)
+            torch.cuda.synchronize()
+            assert (fused[m * (n // 2) :] == -77.0).all()
+            assert np.array_equal(_bits(fused[: m * (n // 2)]), _bits(separate.view(-1)))
+
+
+@pytest.mark.parametrize("rows,full", [(1, 64), (16, 64), (17, 64), (33, 64), (48, 64), (49, 64), (65, 128), (80, 128), (81, 128), (97, 128)])
+def test_decoder_projections_do_not_depend_on_the_batch(device, rows, full):
+    """The projections a decode step issues, at its split counts: a row has the same bits in every batch
+    of 1 to 64 rows, and in every batch of 65 to 128 (between the two the sums are in another order)."""
+    gen = torch.Generator(device=device).manual_seed(rows)
+
+    def weight(n, k):
+        return (torch.randn((n, k), device=device, generator=gen) * 0.02).half()
+
+    fewer = 2 if rows <= dec.GEMM_FEW_ROWS else 1
+    x = torch.randn((full, 2048), device=device, generator=gen).half()
+    wide = torch.randn((full, 5632), device=device, generator=gen).half()
+    products = [
+        (x, weight(2560, 2048), lambda t, w: dec._qkv_projection(t, w)),
+        (x, weight(2048, 2048), lambda t, w: dec._linear_parts(t, w, dec.O_PROJ_SPLITS // fewer)),
+        (wide, weight(2048, 5632), lambda t, w: dec._linear_parts(t, w, dec.DOWN_SPLITS // fewer)),
+        (x, weight(11264, 2048), lambda t, w: dec._swiglu(t, w)),
+    ]
+    for inputs, w, product in products:
+        some, all_rows = product(inputs[:rows].contiguous(), w), product(inputs, w)
+        assert some.shape[:-2] == all_rows.shape[:-2]
+        assert np.array_equal(_bits(some), _bits(all_rows[..., :rows, :]))
+
+
 # --- pc_gemm_rows (a prompt's rows) -----------------------------------------------------------
 
 # (n, k, splits, rows): every tile shape of the dispatch (64 x 64, 128 x 64, 128 x 128,
