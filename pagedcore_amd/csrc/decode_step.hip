@@ -84,6 +84,7 @@ __device__ __forceinline__ half8_t value8(const Chunk8<SPLITS>& c, const void* i
     float4_t lo = c.lo[0], hi = c.hi[0];
     if constexpr (SPLITS == kAnySplits) {
       const float* parts = static_cast<const float*>(input);
+#pragma unroll 4
       for (int s = 1; s < splits; ++s) {
         lo += *reinterpret_cast<const float4_t*>(parts + s * stride + offset);
         hi += *reinterpret_cast<const float4_t*>(parts + s * stride + offset + 4);
@@ -194,9 +195,12 @@ __global__ __launch_bounds__(kRopeThreads) void rope_kv_append_kernel(
 //   h   = fp16(hidden + delta)                     (only when delta is given; stored back)
 //   r   = 1 / sqrt(sum(h * h) / width + eps)       (fp32)
 //   out = fp16(weight * fp16(h * r))
-// Rows of up to 2048 (one chunk per thread) load weight, residual and every part together, with
-// no branch between them: one memory round trip (22 layers of a 7-row MLP 435 -> 414 us, of a
-// 128-row one 731 -> 708).
+// Weight, residual and every part are loaded before the first sum: one memory round trip (22 layers of
+// a 7-row MLP 435 -> 414 us, of a 128-row one 731 -> 708), or one per chunk where the parts of all
+// chunks would take too many registers. Only the last chunk can end inside the row, and threads past
+// it load nothing: with every thread loading four chunks, the row's last one over again, and one
+// part of each at a time, wide rows were slower than with a branch per chunk (us, 8 splits: 37 rows of 2056
+// 5.6, now 3.3, 4.5 with a branch; of 4096 5.6, now 3.4, 4.7; 2048 rows of 2056 35, now 26, 26).
 // ---------------------------------------------------------------------------------------
 
 template <int CTRL>
@@ -219,52 +223,58 @@ __device__ __forceinline__ float wave_sum(float x) {
 }
 
 // delta, when given (HAS_DELTA), is fp16 [rows][width] (SPLITS kFp16Input) or fp32 partial sums
-// [splits][rows][width], rounded to fp16 before the add. CHUNKS chunks per thread. All the
-// parameters fit the 64 bytes that are preloaded into SGPRs.
+// [splits][rows][width], rounded to fp16 before the add. CHUNKS chunks per thread, all but the last
+// within the row for every thread. All the parameters fit the 64 bytes that are preloaded into SGPRs.
 template <int CHUNKS, bool HAS_DELTA, int SPLITS>
 __global__ __launch_bounds__(kNormThreads) void add_rms_norm_kernel(_Float16* hidden, const void* delta,
                                                                     int64_t parts_stride, const _Float16* weight,
                                                                     _Float16* out, int32_t splits, int32_t width,
                                                                     float eps) {
 #pragma clang fp contract(off)
+  // Every chunk's loads at once, or one chunk's at a time where they would take too many registers.
+  constexpr bool kTogether = !HAS_DELTA || CHUNKS * (SPLITS > 0 ? SPLITS : 1) <= 8;
   __shared__ float wave_sums[kNormThreads / 64];
   const int64_t base = static_cast<int64_t>(blockIdx.x) * width;
   const int tid = threadIdx.x;
-  const int chunks = width / 8;
   half8_t wt[CHUNKS], h[CHUNKS];
   Chunk8<SPLITS> d[CHUNKS];
-  int64_t at[CHUNKS];
-  bool mine[CHUNKS];
-#pragma unroll
-  for (int k = 0; k < CHUNKS; ++k) {
-    const int chunk = tid + k * kNormThreads;
-    mine[k] = chunk < chunks;
-    const int safe = mine[k] ? chunk : chunks - 1;  // threads past the row repeat its last chunk
-    at[k] = base + 8 * safe;
-    if constexpr (HAS_DELTA) d[k] = load8<SPLITS>(delta, at[k], parts_stride);
-    h[k] = *reinterpret_cast<const half8_t*>(hidden + at[k]);
-    wt[k] = *reinterpret_cast<const half8_t*>(weight + 8 * safe);
-  }
+  const bool last = tid + (CHUNKS - 1) * kNormThreads < width / 8;
+  auto mine = [&](int k) { return k + 1 < CHUNKS || last; };
+  auto at = [&](int k) { return base + 8 * (tid + k * kNormThreads); };
   float squares = 0.0f;
-#pragma unroll
-  for (int k = 0; k < CHUNKS; ++k) {
+  auto load = [&](int k) {
+    if constexpr (HAS_DELTA) d[k] = load8<SPLITS>(delta, at(k), parts_stride);
+    h[k] = *reinterpret_cast<const half8_t*>(hidden + at(k));
+    wt[k] = *reinterpret_cast<const half8_t*>(weight + 8 * (tid + k * kNormThreads));
+  };
+  auto add = [&](int k) {
     if constexpr (HAS_DELTA) {
-      const half8_t v = value8<SPLITS>(d[k], delta, at[k], parts_stride, splits);
+      const half8_t v = value8<SPLITS>(d[k], delta, at(k), parts_stride, splits);
 #pragma unroll
       for (int i = 0; i < 8; ++i) h[k][i] = round_h(static_cast<float>(h[k][i]) + static_cast<float>(v[i]));
     }
-    if (mine[k]) {
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const float x = static_cast<float>(h[k][i]);
-        squares += x * x;
-      }
+    for (int i = 0; i < 8; ++i) {
+      const float x = static_cast<float>(h[k][i]);
+      squares += x * x;
+    }
+  };
+#pragma unroll
+  for (int k = 0; k < CHUNKS; ++k) {
+    if (mine(k)) load(k);
+    if constexpr (!kTogether) {
+      if (mine(k)) add(k);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+  if constexpr (kTogether) {
+#pragma unroll
+    for (int k = 0; k < CHUNKS; ++k) {
+      if (mine(k)) add(k);
     }
   }
   squares = wave_sum(squares);
   if ((tid & 63) == 0) wave_sums[tid >> 6] = squares;
-  // The barrier also orders every thread's residual loads before the first store: threads past
-  // the row read a chunk that another thread stores.
   __syncthreads();
   float total = 0.0f;
 #pragma unroll
@@ -272,15 +282,15 @@ __global__ __launch_bounds__(kNormThreads) void add_rms_norm_kernel(_Float16* hi
   const float scale = 1.0f / sqrtf(total / static_cast<float>(width) + eps);
 #pragma unroll
   for (int k = 0; k < CHUNKS; ++k) {
-    if (mine[k]) {
+    if (mine(k)) {
       half8_t o;
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
         const float normalized = static_cast<float>(round_h(static_cast<float>(h[k][i]) * scale));
         o[i] = round_h(static_cast<float>(wt[k][i]) * normalized);
       }
-      if constexpr (HAS_DELTA) *reinterpret_cast<half8_t*>(hidden + at[k]) = h[k];
-      *reinterpret_cast<half8_t*>(out + at[k]) = o;
+      if constexpr (HAS_DELTA) *reinterpret_cast<half8_t*>(hidden + at(k)) = h[k];
+      *reinterpret_cast<half8_t*>(out + at(k)) = o;
     }
   }
 }
@@ -359,16 +369,21 @@ int add_rms_norm(void* out, void* hidden, const void* delta, const float* delta_
                        static_cast<_Float16*>(hidden), delta_parts ? static_cast<const void*>(delta_parts) : delta,
                        rows * width, static_cast<const _Float16*>(weight), static_cast<_Float16*>(out), splits, width, eps);
   };
-  const bool one_chunk = width <= kNormThreads * 8;
+  auto launch_row = [&](auto has_delta, auto instance) {
+    constexpr bool D = decltype(has_delta)::value;
+    constexpr int S = decltype(instance)::value;
+    static_assert(kNormMaxChunks == 4, "one instance per chunk count");
+    switch ((width / 8 - 1) / kNormThreads) {
+      case 0: return launch(add_rms_norm_kernel<1, D, S>);
+      case 1: return launch(add_rms_norm_kernel<2, D, S>);
+      case 2: return launch(add_rms_norm_kernel<3, D, S>);
+      default: return launch(add_rms_norm_kernel<4, D, S>);
+    }
+  };
   if (delta == nullptr && delta_parts == nullptr) {
-    one_chunk ? launch(add_rms_norm_kernel<1, false, kFp16Input>) : launch(add_rms_norm_kernel<kNormMaxChunks, false, kFp16Input>);
+    launch_row(std::false_type{}, std::integral_constant<int, kFp16Input>{});
   } else {
-    with_splits(delta_parts == nullptr, splits, [&](auto instance) {
-      constexpr int S = decltype(instance)::value;
-      // Longer rows hold every chunk's parts in registers only one split at a time.
-      if (one_chunk) launch(add_rms_norm_kernel<1, true, S>);
-      else launch(add_rms_norm_kernel<kNormMaxChunks, true, S == kFp16Input ? kFp16Input : kAnySplits>);
-    });
+    with_splits(delta_parts == nullptr, splits, [&](auto instance) { launch_row(std::true_type{}, instance); });
   }
   return check_launch("add_rms_norm");
 }

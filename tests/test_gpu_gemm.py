@@ -371,8 +371,8 @@ def test_gemm_rows_tiles(device, m, n, k, splits):
 # --- the split-K consumers' instances (1, 2, 4, 8 and any other split count; row lengths) ------
 
 
-@pytest.mark.parametrize("splits", [1, 2, 3, 4, 8, 9])
-@pytest.mark.parametrize("rows,width", [(1, 8), (3, 504), (5, 2048), (2, 2056), (3, 8192)])
+@pytest.mark.parametrize("splits", [1, 2, 3, 4, 6, 8, 9])
+@pytest.mark.parametrize("rows,width", [(1, 8), (3, 504), (5, 2048), (2, 2056), (2, 4096), (3, 4104), (2, 5632), (2, 6152), (3, 8192)])
 def test_add_rms_norm_instances(device, rows, width, splits):
     """Parts bit equal to the fp16 path fed their rounded sum, and that path against float64:
     the residual exact, the output within its two fp16 roundings."""
