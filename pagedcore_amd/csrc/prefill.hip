@@ -29,6 +29,10 @@
 // KG = 1): 64 tokens 3.8 -> 3.1, 333 7.3 -> 5.7, 512 9.0 -> 6.9, 1024 14.8 -> 10.6, 2048 31.1 ->
 // 26.5. Slower: three stages (28.7 at 2048, 6.7 at 333), 32 queries per wave (34.2), packed
 // fp16 conversion (29.8 against 28.6).
+//
+// Prompts beyond that keep every SIMD busy whatever the order, and the time is that of the work on a
+// CU: there a workgroup has all eight heads of a kv head (half the staging) and reads K and V two key
+// blocks at a time, which takes 78 registers instead of 96 (24 waves on a CU, not 16 to 20).
 
 #include <hip/hip_runtime.h>
 
@@ -53,9 +57,7 @@ using pc_internal::set_error;
 constexpr int kKVHeads = 4;
 constexpr int kQHeads = 32;
 constexpr int kHeadDim = 64;
-constexpr int kHeads = 4;                    // query heads (waves of a key set) per workgroup
-constexpr int kPerKV = kQHeads / kKVHeads / kHeads;  // workgroups per kv head and query block
-constexpr int kPerBlock = kKVHeads * kPerKV;         // workgroups per query block
+constexpr int kHeadsPerKV = kQHeads / kKVHeads;
 constexpr int kSnake = 256;                  // one workgroup per CU
 constexpr int kBlock = 16;                   // positions per query block and keys per key block
 constexpr int kTileBytes = kBlock * kHeadDim * 2;  // 16 rows of one kv head: 2 KiB
@@ -90,18 +92,22 @@ struct PrefillArgs {
   _Float16* out;
 };
 
-// KG key sets of kHeads waves each. Scalar parameters in the order of PrefillArgs: all are
-// preloaded into SGPRs at wave launch.
-template <int KG>
-__global__ __launch_bounds__(64 * kHeads * KG) void prefill_attention_kernel(const _Float16* q, const _Float16* k,
+// KG key sets of HEADS waves (query heads of one kv head) each. Scalar parameters in the order of
+// PrefillArgs: all are preloaded into SGPRs at wave launch.
+template <int KG, int HEADS>
+__global__ __launch_bounds__(64 * HEADS * KG) void prefill_attention_kernel(const _Float16* q, const _Float16* k,
                                                                              const _Float16* v, int tokens,
                                                                              _Float16* out) {
+  constexpr int kPerKV = kHeadsPerKV / HEADS;   // workgroups per kv head and query block
+  constexpr int kPerBlock = kKVHeads * kPerKV;  // workgroups per query block
+  constexpr int kStagers = HEADS / 4;           // waves that stage the same rows of different key blocks
+  constexpr bool kPairReads = HEADS == 8;       // LDS reads of two key blocks at a time (see the top)
   const PrefillArgs a{q, k, v, tokens, out};
   // Per key set two stages of kStepBlocks key blocks each: stage s, block b: K tile at
   // s * kStageBytes + b * kBufBytes, its V tile kTileBytes after it.
   __shared__ __attribute__((aligned(16))) char smem[KG * 2 * kStageBytes];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int w = wave % kHeads, kg = wave / kHeads;
+  const int w = wave % HEADS, kg = wave / HEADS;
   char* const lds = smem + kg * 2 * kStageBytes;
   const int lane = threadIdx.x & 63;
   const int c = lane & 15;
@@ -119,7 +125,7 @@ __global__ __launch_bounds__(64 * kHeads * KG) void prefill_attention_kernel(con
   }
   const int h = id % kPerBlock / kPerKV;
   const int qb = qblocks - 1 - id / kPerBlock;
-  const int head = kQHeads / kKVHeads * h + kHeads * (id % kPerKV) + w;
+  const int head = kHeadsPerKV * h + HEADS * (id % kPerKV) + w;
   const int pos = kBlock * qb + c;  // this lane's query position (column of S^T)
   const int last = a.tokens - 1;
 
@@ -127,9 +133,9 @@ __global__ __launch_bounds__(64 * kHeads * KG) void prefill_attention_kernel(con
   half8_t qa = *reinterpret_cast<const half8_t*>(qrow);
   half8_t qc = *reinterpret_cast<const half8_t*>(qrow + 32);
 
-  // Staging: wave w of a key set issues kStepBlocks LDS DMA instructions per stage (each 64
-  // lanes x 16 B = rows srow .. srow + 7 of one tile): of every block, the K (w & 2 = 0) or V
-  // tile, rows 8 (w & 1) .. 8 (w & 1) + 7. K piece p of row r sits at position p ^ (r & 7) (the
+  // Staging: wave w of a key set issues kStepBlocks / kStagers LDS DMA instructions per stage (each 64
+  // lanes x 16 B = rows srow .. srow + 7 of one tile): of blocks w / 4, w / 4 + kStagers, ..., the K
+  // (w & 2 = 0) or V tile, rows 8 (w & 1) .. 8 (w & 1) + 7. K piece p of row r sits at position p ^ (r & 7) (the
   // A-operand reads of 16 rows then hit 8 different 16 B bank groups); V uses the decode
   // kernel's 32 B-group swizzle for its transposing reads.
   const bool stage_v = (w & 2) != 0;
@@ -152,7 +158,8 @@ __global__ __launch_bounds__(64 * kHeads * KG) void prefill_attention_kernel(con
   // repeat its last row; their scores are masked).
   auto stage = [&](int j, int buf) {
 #pragma unroll
-    for (int b = 0; b < kStepBlocks; ++b) {
+    for (int i = 0; i < kStepBlocks / kStagers; ++i) {
+      const int b = w / 4 + kStagers * i;
       const int row = min(kBlock * (kStepBlocks * j + b) + srow, last);
       __builtin_amdgcn_global_load_lds(static_cast<const void*>(ssrc + static_cast<int64_t>(row) * kKVHeads * kHeadDim),
                                        lds_ptr(lds + buf * kStageBytes + sdst + b * kBufBytes), 16, 0, 0);
@@ -187,7 +194,28 @@ __global__ __launch_bounds__(64 * kHeads * KG) void prefill_attention_kernel(con
     if (KG > 1 && j >= steps) return;  // the last round of a set with no step left in it
     // sc[4 b + e]: key 4g + e of block kStepBlocks * j + b
     float sc[4 * kStepBlocks];
-    {
+    if constexpr (kPairReads) {
+      for_pairs([&](auto pair) {
+        constexpr int b = 2 * decltype(pair)::value;
+        half8_t k00, k01, k10, k11;
+        asm volatile(
+            "ds_read_b128 %0, %4 offset:%6\n\tds_read_b128 %1, %5 offset:%6\n\tds_read_b128 %2, %4 offset:%7\n\t"
+            "ds_read_b128 %3, %5 offset:%7\n\ts_waitcnt lgkmcnt(0)"
+            : "=&v"(k00), "=&v"(k01), "=&v"(k10), "=&v"(k11)
+            : "v"(kaddr0), "v"(kaddr1), "i"(so + b * kBufBytes), "i"(so + (b + 1) * kBufBytes)
+            : "memory");
+        float4_t s0 = {0.f, 0.f, 0.f, 0.f}, s1 = {0.f, 0.f, 0.f, 0.f};
+        s0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(k00, qa, s0, 0, 0, 0);
+        s1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(k10, qa, s1, 0, 0, 0);
+        s0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(k01, qc, s0, 0, 0, 0);
+        s1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(k11, qc, s1, 0, 0, 0);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          sc[4 * b + e] = s0[e];
+          sc[4 * b + 4 + e] = s1[e];
+        }
+      });
+    } else     {
       half8_t kf[8];
       asm volatile(
           "ds_read_b128 %0, %8 offset:%10\n\tds_read_b128 %1, %9 offset:%10\n\t"
@@ -236,37 +264,52 @@ __global__ __launch_bounds__(64 * kHeads * KG) void prefill_attention_kernel(con
       mc = m * kScoreToLog2;
     }
     __builtin_amdgcn_sched_barrier(0);
-    short4_t vt[16];  // vt[4 b + u]: block b, dims 16 u .. 16 u + 15
-    asm volatile(
-        "ds_read_b64_tr_b16 %0, %16 offset:%20\n\tds_read_b64_tr_b16 %1, %17 offset:%20\n\t"
-        "ds_read_b64_tr_b16 %2, %18 offset:%20\n\tds_read_b64_tr_b16 %3, %19 offset:%20\n\t"
-        "ds_read_b64_tr_b16 %4, %16 offset:%21\n\tds_read_b64_tr_b16 %5, %17 offset:%21\n\t"
-        "ds_read_b64_tr_b16 %6, %18 offset:%21\n\tds_read_b64_tr_b16 %7, %19 offset:%21\n\t"
-        "ds_read_b64_tr_b16 %8, %16 offset:%22\n\tds_read_b64_tr_b16 %9, %17 offset:%22\n\t"
-        "ds_read_b64_tr_b16 %10, %18 offset:%22\n\tds_read_b64_tr_b16 %11, %19 offset:%22\n\t"
-        "ds_read_b64_tr_b16 %12, %16 offset:%23\n\tds_read_b64_tr_b16 %13, %17 offset:%23\n\t"
-        "ds_read_b64_tr_b16 %14, %18 offset:%23\n\tds_read_b64_tr_b16 %15, %19 offset:%23\n\t"
-        "s_waitcnt lgkmcnt(0)"
-        : "=&v"(vt[0]), "=&v"(vt[1]), "=&v"(vt[2]), "=&v"(vt[3]), "=&v"(vt[4]), "=&v"(vt[5]), "=&v"(vt[6]),
-          "=&v"(vt[7]), "=&v"(vt[8]), "=&v"(vt[9]), "=&v"(vt[10]), "=&v"(vt[11]), "=&v"(vt[12]), "=&v"(vt[13]),
-          "=&v"(vt[14]), "=&v"(vt[15])
-        : "v"(va[0]), "v"(va[1]), "v"(va[2]), "v"(va[3]), "i"(so), "i"(so + kBufBytes), "i"(so + 2 * kBufBytes),
-          "i"(so + 3 * kBufBytes)
-        : "memory");
     // Per pair of blocks, P^T as one 32-key B operand: element e is key 4g + (e & 3) of
     // the pair's block e / 4; the V^T A operands concatenate the two blocks in the same
     // order.
-    auto accumulate = [&](auto pair) {
-      constexpr int b = 2 * decltype(pair)::value;
+    auto weights = [&](int b) {
       half8_t pb;
 #pragma unroll
       for (int e = 0; e < 8; ++e) pb[e] = static_cast<_Float16>(exp2_fast(fmaf(sc[4 * b + e], kScoreToLog2, -mc)));
+      return pb;
+    };
+    auto accumulate = [&](const half8_t pb, const short4_t* v0, const short4_t* v1) {
 #pragma unroll
-      for (int u = 0; u < 4; ++u)
-        acc[u] = __builtin_amdgcn_mfma_f32_16x16x32_f16(join(vt[4 * b + u], vt[4 * b + 4 + u]), pb, acc[u], 0, 0, 0);
+      for (int u = 0; u < 4; ++u) acc[u] = __builtin_amdgcn_mfma_f32_16x16x32_f16(join(v0[u], v1[u]), pb, acc[u], 0, 0, 0);
       lacc = __builtin_amdgcn_mfma_f32_16x16x32_f16(ones, pb, lacc, 0, 0, 0);
     };
-    for_pairs(accumulate);
+    if constexpr (kPairReads) {
+      for_pairs([&](auto pair) {
+        constexpr int b = 2 * decltype(pair)::value;
+        const half8_t pb = weights(b);
+        short4_t v0[4], v1[4];
+        read_v_tiles<so + b * kBufBytes>(vbase, tsel, v0[0], v0[1], v0[2], v0[3]);
+        read_v_tiles<so + (b + 1) * kBufBytes>(vbase, tsel, v1[0], v1[1], v1[2], v1[3]);
+        accumulate(pb, v0, v1);
+      });
+    } else {
+      short4_t vt[16];  // vt[4 b + u]: block b, dims 16 u .. 16 u + 15
+      asm volatile(
+          "ds_read_b64_tr_b16 %0, %16 offset:%20\n\tds_read_b64_tr_b16 %1, %17 offset:%20\n\t"
+          "ds_read_b64_tr_b16 %2, %18 offset:%20\n\tds_read_b64_tr_b16 %3, %19 offset:%20\n\t"
+          "ds_read_b64_tr_b16 %4, %16 offset:%21\n\tds_read_b64_tr_b16 %5, %17 offset:%21\n\t"
+          "ds_read_b64_tr_b16 %6, %18 offset:%21\n\tds_read_b64_tr_b16 %7, %19 offset:%21\n\t"
+          "ds_read_b64_tr_b16 %8, %16 offset:%22\n\tds_read_b64_tr_b16 %9, %17 offset:%22\n\t"
+          "ds_read_b64_tr_b16 %10, %18 offset:%22\n\tds_read_b64_tr_b16 %11, %19 offset:%22\n\t"
+          "ds_read_b64_tr_b16 %12, %16 offset:%23\n\tds_read_b64_tr_b16 %13, %17 offset:%23\n\t"
+          "ds_read_b64_tr_b16 %14, %18 offset:%23\n\tds_read_b64_tr_b16 %15, %19 offset:%23\n\t"
+          "s_waitcnt lgkmcnt(0)"
+          : "=&v"(vt[0]), "=&v"(vt[1]), "=&v"(vt[2]), "=&v"(vt[3]), "=&v"(vt[4]), "=&v"(vt[5]), "=&v"(vt[6]),
+            "=&v"(vt[7]), "=&v"(vt[8]), "=&v"(vt[9]), "=&v"(vt[10]), "=&v"(vt[11]), "=&v"(vt[12]), "=&v"(vt[13]),
+            "=&v"(vt[14]), "=&v"(vt[15])
+          : "v"(va[0]), "v"(va[1]), "v"(va[2]), "v"(va[3]), "i"(so), "i"(so + kBufBytes), "i"(so + 2 * kBufBytes),
+            "i"(so + 3 * kBufBytes)
+          : "memory");
+      for_pairs([&](auto pair) {
+        constexpr int b = 2 * decltype(pair)::value;
+        accumulate(weights(b), vt + 4 * b, vt + 4 * b + 4);
+      });
+    }
   };
 
   if (kg < steps) stage(kg, 0);
@@ -327,13 +370,18 @@ extern "C" int pc_prefill_attention(void* out, const void* query, const void* ke
     return set_error(PC_ERR_ARGUMENT, "buffers must be 16-byte aligned");
   // Two key sets while their workgroups (64 KiB of LDS, two per CU) run at once, above the 128
   // tokens (two steps) where the merge costs more than the shorter chain saves: 3.8 against
-  // 4.1 us at 128 tokens, 5.1 / 5.1 at 256, 6.1 / 5.7 at 333, 12.3 / 10.6 at 1024, 15.3 / 15.3
-  // at 1280, 26.5 / 29.6 at 2048.
-  const unsigned grid = static_cast<unsigned>((tokens + kBlock - 1) / kBlock) * kPerBlock;
-  const bool split = tokens > 128 && grid <= 2 * kSnake;
-  auto kernel = split ? prefill_attention_kernel<2> : prefill_attention_kernel<1>;
-  hipLaunchKernelGGL(kernel, dim3(grid), dim3(64 * kHeads * (split ? 2 : 1)), 0, static_cast<hipStream_t>(stream),
-                     static_cast<const _Float16*>(query), static_cast<const _Float16*>(key),
-                     static_cast<const _Float16*>(value), static_cast<int>(tokens), static_cast<_Float16*>(out));
+  // 4.1 us at 128 tokens, 5.1 / 5.1 at 256, 6.1 / 5.7 at 333, 12.3 / 10.6 at 1024, 26.5 / 29.6
+  // at 2048. Eight heads per workgroup from the sixth round of half-size ones on, where what counts is
+  // the waves on a CU and the bytes staged, no longer how evenly the CUs end (us against four heads):
+  // 33.4 / 31.4 at 2300 tokens, 40.2 / 41.1 at 2600, 49.6 / 52.6 at 3000, 89.7 / 93.3 at 4096, 323 / 352 at 8192.
+  const unsigned blocks = static_cast<unsigned>((tokens + kBlock - 1) / kBlock);
+  auto launch = [&](auto kernel, unsigned per_block, int waves) {
+    hipLaunchKernelGGL(kernel, dim3(blocks * per_block), dim3(64 * waves), 0, static_cast<hipStream_t>(stream),
+                       static_cast<const _Float16*>(query), static_cast<const _Float16*>(key),
+                       static_cast<const _Float16*>(value), static_cast<int>(tokens), static_cast<_Float16*>(out));
+  };
+  if (8 * blocks > 5 * kSnake) launch(prefill_attention_kernel<1, 8>, 4, 8);
+  else if (tokens > 128 && 8 * blocks <= 2 * kSnake) launch(prefill_attention_kernel<2, 4>, 8, 8);
+  else launch(prefill_attention_kernel<1, 4>, 8, 4);
   return check_launch("prefill_attention");
 }

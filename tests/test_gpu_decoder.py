@@ -711,9 +711,9 @@ def _causal_fp64_on(query, key, value):
 
 
 @pytest.mark.parametrize("sharp", [False, True])
-@pytest.mark.parametrize("tokens", [112, 128, 129, 193, 1023, 1024, 1025, 2047, 4100])
+@pytest.mark.parametrize("tokens", [112, 128, 129, 193, 1023, 1024, 1025, 2047, 2560, 2561, 4100])
 def test_prefill_attention_at_the_dispatch_edges(device, tokens, sharp):
-    """Both forms of the kernel (one and two key sets) on either side of the sizes where they
+    """The forms of the kernel (one and two key sets, eight heads) on either side of the sizes where they
     change, a last chunk of workgroups that is partly filled, and more than eight chunks;
     unit and +-1000-scale scores, against FP64 within the kernel's 2e-3."""
     gen = torch.Generator(device=device).manual_seed(tokens + sharp)
