@@ -31,7 +31,7 @@ enum pc_status {
   PC_ERR_LAUNCH = 2,   /* the HIP runtime rejected a kernel launch */
 };
 
-/* ABI revision; bumped whenever a signature or a layout contract changes. */
+/* ABI revision; bumped whenever an entry point is added or a signature or a layout contract changes. */
 int pc_abi_version(void);
 
 /* Text describing the last failure on the calling thread ("" if none). */

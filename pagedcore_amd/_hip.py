@@ -17,7 +17,7 @@ import numpy as np
 import torch
 from torch import Tensor
 
-ABI_VERSION = 13
+ABI_VERSION = 14
 LIBRARY_NAME = "libpagedcore_hip.so"
 
 _lock = threading.Lock()
@@ -103,8 +103,6 @@ def library_path() -> str:
 
 
 def _declare(lib: ctypes.CDLL) -> None:
-    lib.pc_abi_version.restype = ctypes.c_int
-    lib.pc_abi_version.argtypes = []
     lib.pc_last_error.restype = ctypes.c_char_p
     lib.pc_last_error.argtypes = []
     lib.pc_attn_workspace_bytes.restype = _i64
@@ -162,10 +160,16 @@ def load() -> ctypes.CDLL:
                 lib = ctypes.CDLL(path)
             except OSError as error:
                 raise HipExtensionError(f"cannot load {path}: {error}") from error
-            _declare(lib)
-            version = lib.pc_abi_version()
+            # The version first: a library of another one may lack what _declare names.
+            try:
+                lib.pc_abi_version.restype = ctypes.c_int
+                lib.pc_abi_version.argtypes = []
+                version = lib.pc_abi_version()
+            except AttributeError as error:
+                raise HipExtensionError(f"{path} is not this library: {error}") from error
             if version != ABI_VERSION:
                 raise HipExtensionError(f"{path} has ABI {version}, expected {ABI_VERSION}")
+            _declare(lib)
             _library = lib
     return _library
 

@@ -6,6 +6,7 @@ from __future__ import annotations
 import ctypes
 import os
 import re
+import subprocess
 
 import numpy as np
 import pytest
@@ -235,6 +236,19 @@ def test_decode_plan_rejects_bad_arguments():
         assert b"exceeds its 16-block table" in lib.pc_last_error()
     lens[1] = 16 * 16
     assert plan(lens.ctypes.data, tables.ctypes.data, 2, 16, records.ctypes.data, 64) == 8
+
+
+@pytest.mark.parametrize("source,needle", [("int pc_abi_version(void) { return 13; }", "has ABI 13, expected"), ("int other(void) { return 0; }", "pc_abi_version")])
+def test_a_library_of_another_abi_is_refused_by_its_version(monkeypatch, tmp_path, source, needle):
+    """A library that lacks entry points of this binding is named by its version, not by the first
+    symbol it lacks."""
+    stub, library = tmp_path / "stub.c", tmp_path / "stub.so"
+    stub.write_text(source)
+    subprocess.run(["gcc", "-shared", "-fPIC", "-o", str(library), str(stub)], check=True)
+    monkeypatch.setattr(_hip, "_library", None)
+    monkeypatch.setattr(_hip, "library_path", lambda: str(library))
+    with pytest.raises(_hip.HipExtensionError, match=needle):
+        _hip.load()
 
 
 def test_missing_library_fails_loudly(monkeypatch, tmp_path):
