@@ -1,6 +1,6 @@
 // Device helpers shared by the library's kernels (not part of the C ABI): vector types,
-// cross-lane reductions over the four 16-lane groups of a wave, loads issued without
-// compiler tracking, and the transposing LDS reads of 16-token V tiles.
+// cross-lane reductions over the four 16-lane groups of a wave, and the transposing LDS reads
+// of 16-token V tiles.
 #ifndef PAGEDCORE_PC_DEVICE_H
 #define PAGEDCORE_PC_DEVICE_H
 
@@ -12,9 +12,7 @@ namespace pc_device {
 
 typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
 typedef _Float16 half4_t __attribute__((ext_vector_type(4)));
-typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
 typedef float float4_t __attribute__((ext_vector_type(4)));
-typedef float float2_t __attribute__((ext_vector_type(2)));
 typedef short short4_t __attribute__((ext_vector_type(4)));
 typedef uint32_t uint2_t __attribute__((ext_vector_type(2)));
 
@@ -70,39 +68,12 @@ __device__ __forceinline__ void read_v_tiles(uint32_t base, uint32_t sel, short4
       : "memory");
 }
 
-// 16 B at p and p + 64 B, issued without compiler tracking; wait_loads<N>() on the same
-// registers (N = loads issued after them) makes them available.
-__device__ __forceinline__ void load_pair(half8_t& x, half8_t& y, const _Float16* p) {
-  asm volatile("global_load_dwordx4 %0, %2, off\n\tglobal_load_dwordx4 %1, %2, off offset:64"
-               : "=&v"(x), "=&v"(y)
-               : "v"(p)
-               : "memory");
-}
-
 // Cache policy of loads that stream data read once per pass (the KV pool, decode weights):
 // non-temporal (`nt`). Such streams are far larger than the caches; allocating them there
 // only costs bandwidth (a load-only pass over the paged KV layout measured 11.9 us with `nt`
 // against 13.2 us with the default policy, on the VGPR and the LDS DMA path alike).
 // kStreamAux is the same bit as the cache-policy operand of __builtin_amdgcn_global_load_lds.
 constexpr int kStreamAux = 2;
-
-// load_pair with the streaming policy.
-__device__ __forceinline__ void load_pair_stream(half8_t& x, half8_t& y, const _Float16* p) {
-  asm volatile("global_load_dwordx4 %0, %2, off nt\n\tglobal_load_dwordx4 %1, %2, off offset:64 nt"
-               : "=&v"(x), "=&v"(y)
-               : "v"(p)
-               : "memory");
-}
-
-template <int N>
-__device__ __forceinline__ void wait_loads(half8_t& x, half8_t& y) {
-  asm volatile("s_waitcnt vmcnt(%2)" : "+v"(x), "+v"(y) : "i"(N) : "memory");
-}
-
-template <int N>
-__device__ __forceinline__ void wait_loads4(half8_t& x, half8_t& y, half8_t& z, half8_t& t) {
-  asm volatile("s_waitcnt vmcnt(%4)" : "+v"(x), "+v"(y), "+v"(z), "+v"(t) : "i"(N) : "memory");
-}
 
 }  // namespace pc_device
 
