@@ -53,13 +53,18 @@ FLAGS = [
     "-Rpass-analysis=kernel-resource-usage",
 ]
 
-# Kernels checked after every build: (demangled-name fragment) -> minimum waves per SIMD
-# the kernel's launch shape relies on. Each must report no scratch and no spills.
+# Kernels checked after every build: (fragment of the mangled name) -> minimum waves per SIMD
+# the kernel's launch shape relies on. Each must report no scratch and no spills. A fragment
+# without template arguments holds for every instance of the kernel; one with them names the
+# instance whose workgroups are meant to share a CU.
 GUARDED_KERNELS: Dict[str, int] = {
     "paged_decode_bin_kernel": 2,
-    "prefill_attention_kernel": 4,
-    "gemm_stream_kernel": 1,
-    "gemm_tile_kernel": 1,
+    "prefill_attention_kernel": 4,  # two workgroups of eight waves, four of four
+    "prefill_attention_kernelILi1ELi8E": 6,  # three workgroups of eight waves
+    "gemm_stream_kernel": 2,  # two workgroups of four waves (up to 80 KB of LDS each)
+    "gemm_stream_kernelILi1ELi2ELi4ELi2E": 3,  # three (48 KB)
+    "gemm_tile_kernel": 2,  # a workgroup of eight waves
+    "gemm_tile_kernelILi128ELi192ELi4ELi2ELi2E": 4,  # two of them (80 KB): SwiGLU of long prompts
 }
 
 _NOISE = "packed-fp32-ops' is not a recognized feature"

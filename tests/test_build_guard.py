@@ -91,3 +91,14 @@ def test_the_library_kernels_pass_the_check(tmp_path):
     summary = build.check_resource_usage(text)
     assert len(summary) >= len(build.GUARDED_KERNELS)
     assert all("scratch 0 B, spills 0/0" in line for line in summary)
+    # A guarded instance that loses one wave per SIMD (one register too many) is refused, also where
+    # the kernel's other instances need fewer.
+    for fragment in (name for name in build.GUARDED_KERNELS if "ILi" in name):
+        name, fields = next((n, f) for n, f in build.parse_resource_usage(text).items() if fragment in n)
+        needed = build.GUARDED_KERNELS[fragment]
+        report = text.split(f"Function Name: {name} ")
+        waves = f"Occupancy [waves/SIMD]: {fields['Occupancy [waves/SIMD]']}"
+        assert len(report) == 2 and waves in report[1]
+        lower = report[1].replace(waves, f"Occupancy [waves/SIMD]: {needed - 1}", 1)
+        with pytest.raises(build.ResourceCheckError, match="waves/SIMD its launch shape assumes"):
+            build.check_resource_usage(f"Function Name: {name} ".join((report[0], lower)))
