@@ -294,13 +294,19 @@ def _kernel_operands(x: Tensor, weight: Tensor) -> bool:
     )
 
 
+def _rows_fit(rows: int, n: int, k: int, splits: int = 1) -> bool:
+    """Whether the product lies within the sizes that pc_gemm_rows takes."""
+    return rows <= 65536 and k <= 1 << 22 and max(rows * k, n * k, splits * rows * n) <= 1 << 31
+
+
 def _linear_rows(x: Tensor, weight: Tensor) -> Tensor:
     """x @ weight.T above GEMM_M128_ROWS rows: fp32 partial sums or the fp16 product of
     pc_gemm_rows, or F.linear where that is faster or the shape does not fit the kernel."""
     rows, k = x.shape
     n = weight.shape[0]
     splits = _rows_splits(rows, n, k)
-    if splits and n % 32 == 0 and k % (64 * splits) == 0 and _kernel_operands(x, weight):
+    fits = splits and n % 32 == 0 and k % (64 * splits) == 0 and _rows_fit(rows, n, k, splits)
+    if fits and _kernel_operands(x, weight):
         if splits > 1:
             parts = torch.empty((splits, rows, n), dtype=torch.float32, device=x.device)
             _hip.gemm_rows(parts, x, weight, splits=splits)
@@ -372,7 +378,7 @@ def _swiglu(x: Tensor, gate_up: Tensor) -> Tensor:
     rows, k = x.shape
     n = gate_up.shape[0]
     activated = torch.empty((rows, n // 2), dtype=torch.float16, device=x.device)
-    fits = n % 64 == 0 and k % 64 == 0 and _kernel_operands(x, gate_up)
+    fits = n % 64 == 0 and k % 64 == 0 and _rows_fit(rows, n, k) and _kernel_operands(x, gate_up)
     if fits and rows <= GEMM_M128_ROWS:
         _hip.gemm_m128(activated, x, gate_up, epilogue=_hip.GEMM_SWIGLU)
     elif fits and _rows_swiglu(rows, n // 2):

@@ -239,6 +239,19 @@ def test_projection_route_takes_only_what_the_kernels_read(monkeypatch, rows, fo
         torch.testing.assert_close(fused, expected, atol=4e-3 * expected.abs().max().item(), rtol=0)
 
 
+@pytest.mark.parametrize("rows,width,k,taken", [(65536, 5632, 64, True), (65537, 5632, 64, False), (40000, 28672, 64, False)])
+def test_swiglu_beyond_the_kernels_sizes_is_the_librarys(monkeypatch, rows, width, k, taken):
+    """More rows, or more output elements, than pc_gemm_rows takes go to F.linear and pc_silu_mul, as
+    every row count above 128 did before that kernel."""
+    calls = []
+    monkeypatch.setattr(_hip, "gemm_rows", lambda out, x, w, **options: calls.append("rows"))
+    monkeypatch.setattr(_hip, "silu_mul", lambda out, gate_up: calls.append("library"))
+    monkeypatch.setattr(torch.nn.functional, "linear", lambda x, w: None)
+    monkeypatch.setattr(dec, "_rows_swiglu", lambda rows, width: True)
+    dec._swiglu(torch.empty((rows, k), dtype=torch.float16), torch.empty((2 * width, k), dtype=torch.float16))
+    assert calls == (["rows"] if taken else ["library"])
+
+
 @pytest.mark.parametrize("n,k", [(2560, 2048), (2048, 2048), (2048, 5632), (32000, 2048), (128, 64)])
 def test_rows_splits_always_divide_into_the_decoders_shapes(n, k):
     for rows in range(129, 2049):
