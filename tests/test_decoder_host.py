@@ -252,11 +252,21 @@ def test_swiglu_beyond_the_kernels_sizes_is_the_librarys(monkeypatch, rows, widt
     assert calls == (["rows"] if taken else ["library"])
 
 
-@pytest.mark.parametrize("n,k", [(2560, 2048), (2048, 2048), (2048, 5632), (32000, 2048), (128, 64)])
+@pytest.mark.parametrize("n,k", [(2560, 2048), (2048, 2048), (2048, 5632), (32000, 2048)])
 def test_rows_splits_always_divide_into_the_decoders_shapes(n, k):
     for rows in range(129, 2049):
         splits = dec._rows_splits(rows, n, k)
         assert splits in (0, 1, 2, 4)
+        if splits:
+            assert k % (64 * splits) == 0
         if splits > 1:
             # the partials stay a fraction of the weight they save reading late
             assert splits * rows * n * 4 <= 32 << 20
+
+
+def test_rows_whose_k_does_not_divide_are_the_librarys(monkeypatch):
+    """K of one unit cannot be split in two, the count the rule names at this size."""
+    assert dec._rows_splits(129, 128, 64) == 2
+    monkeypatch.setattr(_hip, "gemm_rows", lambda *args, **options: pytest.fail("not divisible"))
+    x, weight = torch.ones((129, 64), dtype=torch.float16), torch.ones((128, 64), dtype=torch.float16)
+    assert torch.equal(dec._linear_parts(x, weight, 4), torch.nn.functional.linear(x, weight))

@@ -230,6 +230,29 @@ def test_prefill_paged_matches_the_contiguous_prefill(device, lengths):
         assert torch.equal(after[:, :, others].isnan(), before[:, :, others].isnan())
 
 
+@pytest.mark.parametrize("tokens", [300, 600, 1000])
+def test_long_prefill_with_the_full_mlp_width_is_as_accurate_as_the_reference(device, tokens):
+    """Prompts on every route of the projections above 128 rows (o_proj at 2 splits, by the library and
+    unsplit, down at 4 and 2, SwiGLU tiles), with the model's MLP of 5632: logits and the
+    cached K/V of every layer are as close to the fp32 forward as the reference's own fp16 forward
+    is (both evaluated by the oracle's torch expressions on the GPU, attention in fp32)."""
+    small = dec.random_weights(device=device, seed=tokens, layers=2, vocab=31, norm_std=0.1)
+    weights = dec.TinyLlamaWeights(small.embedding, small.layers * 11, small.final_norm, small.lm_head)
+    allocator = KVAllocator(torch.zeros((22, 2, 64, 16, 4, 64), dtype=torch.float16, device=device))
+    request = RequestId("long")
+    allocator.create(KVReservation(request, (tokens + 15) // 16))
+    ids = torch.randint(0, 31, (1, tokens), device=device)
+    logits = dec.prefill_paged(ids, weights, allocator, request)
+    with torch.inference_mode(), torch.device(device):
+        half_logits, half_cache = dref.forward(ids, weights, fp32_attention=True)
+        exact_logits, exact_cache = dref.forward(ids, _fp32(weights), fp32_attention=True)
+    _as_accurate(logits, half_logits, exact_logits)
+    got = _pool_cache(allocator, request)
+    for layer in range(22):
+        for kind in range(2):
+            _as_accurate(got[layer][kind], half_cache[layer][kind], exact_cache[layer][kind])
+
+
 @pytest.mark.parametrize("lengths", [(15,), (1, 15, 16, 17, 49)])
 def test_decode_paged_matches_the_contiguous_fp32_decode(device, lengths):
     """tests/unit/test_decoder.py:114-195: two steps (the second in reverse request order);
@@ -1088,7 +1111,8 @@ def test_worker_streams_match_the_oracle_generate(device, graph_batch, prompt_gr
 @pytest.mark.parametrize("batch,expect_library_gemm", [(128, True), (130, False)])
 def test_decode_paged_projection_path_by_batch_size(device, monkeypatch, batch, expect_library_gemm):
     """Up to 128 rows the step's projections run on pc_gemm_m128 (split-K partials summed by
-    the RoPE / residual kernels, SwiGLU fused); above that on F.linear. Both paths match the
+    the RoPE / residual kernels, SwiGLU fused); above that none does: q|k|v, o_proj and gate|up run
+    on pc_gemm_rows (unsplit fp16, 2 splits, SwiGLU). Both paths match the
     contiguous fp32 decode (tests/unit/test_decoder.py:114-195 tolerances) on sampled rows."""
     weights = _synthetic(device)
     host_weights = _cpu(weights)
@@ -1108,6 +1132,14 @@ def test_decode_paged_projection_path_by_batch_size(device, monkeypatch, batch, 
         return original(*args, **kwargs)
 
     monkeypatch.setattr(_hip, "gemm_m128", counting)
+    rows_calls = []
+    original_rows = _hip.gemm_rows
+
+    def counting_rows(*args, **kwargs):
+        rows_calls.append((kwargs.get("epilogue", _hip.GEMM_PARTIALS), kwargs.get("splits", 1)))
+        return original_rows(*args, **kwargs)
+
+    monkeypatch.setattr(_hip, "gemm_rows", counting_rows)
     tokens = torch.tensor([[(5 * row) % 31] for row in range(batch)])
     sample = [0, 1, 2, batch // 2, batch - 1]
     expected = {row: dref.decode_fp32(tokens[row : row + 1], _pool_cache(allocator, requests[row]), host_weights)
@@ -1118,8 +1150,10 @@ def test_decode_paged_projection_path_by_batch_size(device, monkeypatch, batch, 
         # per layer q|k|v, o_proj and gate|up (the synthetic MLP width 32 keeps down, whose
         # K of 32 is not a multiple of 64, on F.linear)
         assert calls.count(_hip.GEMM_PARTIALS) == 2 * 22 and calls.count(_hip.GEMM_SWIGLU) == 22
+        assert rows_calls == []
     else:
         assert calls == []
+        assert rows_calls == 22 * [(_hip.GEMM_HALF, 1), (_hip.GEMM_PARTIALS, 2), (_hip.GEMM_SWIGLU, 1)]
     assert torch.isfinite(logits).all()
     for row in sample:
         torch.testing.assert_close(logits[row : row + 1].cpu(), expected[row][0], atol=5e-3, rtol=5e-3)

@@ -322,9 +322,10 @@ def test_decoder_projections_do_not_depend_on_the_batch(device, rows, full):
 
 # --- pc_gemm_rows (a prompt's rows) -----------------------------------------------------------
 
-# (n, k, splits, rows): every tile shape of the dispatch (64 x 64, 128 x 64, 128 x 128,
-# 128 x 192; SwiGLU 48, 96 and 128 output columns, and 96 on two stages), rows one short of, at
-# and one past a tile, column counts that end inside a tile, fewer K stages than the ring has.
+# (n, k, splits, rows): every tile shape of the dispatch under every epilogue that reaches it (64 x 64,
+# 128 x 64, 128 x 128, 128 x 192; SwiGLU 48, 96 and 128 output columns, and 96 on two stages; the
+# streams of an unsplit product of few columns), rows one short of, at and one past a tile, column
+# counts that end inside a tile, fewer K stages than the ring has, and the decoder's own shapes.
 ROWS_SHAPES = [
     (64, 64, 1, (1, 63, 64, 65, 200)),
     (352, 128, 1, (129, 255)),
@@ -332,14 +333,18 @@ ROWS_SHAPES = [
     (2048, 5632, 4, (129, 300, 513)),
     (2080, 1408, 2, (641, 1025)),
     (11264, 256, 1, (129, 300, 600, 700)),
+    (2048, 2048, 1, (257, 288, 289, 385, 512, 513, 897, 1023, 1024, 1025)),
+    (2560, 2048, 1, (145, 289, 769, 1536, 1537)),
+    (2048, 5632, 2, (769, 1024)),
+    (11264, 2048, 1, (256, 257, 513, 640, 641, 1409)),
 ]
 
 
 @pytest.mark.parametrize("n,k,splits,m", [(n, k, s, m) for n, k, s, rows in ROWS_SHAPES for m in rows])
 def test_gemm_rows_tiles(device, m, n, k, splits):
-    """Partials against fp32 split by split, nothing written past the output; with one split the
-    fp16 epilogue bit equal to the rounded partials, and SwiGLU within the rounding of its
-    two projections of pc_silu_mul of them (its tiles may differ, the K order does not)."""
+    """Partials against float64 split by split, nothing written past the output; with one split the
+    fp16 epilogue bit equal to the rounded partials, and SwiGLU bit equal to pc_silu_mul of its
+    two projections (its tiles may differ, the K order does not)."""
     x, w = _inputs(device, m, n, k, seed=5 * m + n + k)
     guard = torch.full((splits * m * n + 64,), -77.0, dtype=torch.float32, device=device)
     out = guard[: splits * m * n].view(splits, m, n).fill_(float("nan"))

@@ -321,6 +321,44 @@ def test_gemm_rejects_invalid_arguments_without_a_gpu(overrides, needle):
 @pytest.mark.parametrize(
     "overrides,needle",
     [
+        ({"out": None}, b"null pointer"),
+        ({"w": None}, b"null pointer"),
+        ({"m": 0}, b"m = 0"),
+        ({"m": 65537}, b"65536"),
+        ({"n": 0}, b"must be positive"),
+        ({"k": -64}, b"must be positive"),
+        ({"splits": 0}, b"must be positive"),
+        ({"splits": 3}, b"not divisible"),
+        ({"k": 96, "splits": 1}, b"multiple of 64"),
+        ({"k": 2048, "splits": 64}, b"multiple of 64"),
+        ({"k": (1 << 22) + 64, "n": 32, "m": 1, "splits": 1}, b"too large"),
+        ({"n": 1 << 20, "k": 1 << 12}, b"too large"),
+        ({"m": 65536, "k": 1 << 16, "n": 32, "splits": 1}, b"too large"),
+        ({"m": 65536, "n": 1 << 14}, b"too large"),
+        ({"out": 264}, b"aligned"),
+        ({"x": 264}, b"aligned"),
+        ({"w": 264}, b"aligned"),
+        ({"n": 48}, b"multiple of 32"),
+        ({"epilogue": 1, "splits": 2}, b"one split"),
+        ({"epilogue": 2, "splits": 2}, b"one split"),
+        ({"epilogue": 2, "n": 96, "splits": 1}, b"multiple of 64"),
+        ({"epilogue": 3, "splits": 1}, b"unknown epilogue"),
+        ({"epilogue": 7}, b"unknown epilogue"),
+    ],
+)
+def test_gemm_rows_rejects_invalid_arguments_without_a_gpu(overrides, needle):
+    """pc_gemm_rows validates shapes, splits, epilogue and alignment before any HIP call."""
+    lib = _hip.load()
+    a = {"out": 256, "x": 256, "w": 256, "m": 512, "n": 2048, "k": 2048, "splits": 4, "epilogue": 0}
+    a.update(overrides)
+    status = lib.pc_gemm_rows(a["out"], a["x"], a["w"], a["m"], a["n"], a["k"], a["splits"], a["epilogue"], None)
+    assert status == 1
+    assert needle in lib.pc_last_error()
+
+
+@pytest.mark.parametrize(
+    "overrides,needle",
+    [
         ({"query": None}, b"null pointer"),
         ({"w": None}, b"null pointer"),
         ({"m": 0}, b"m = 0"),
