@@ -261,25 +261,29 @@ DOWN_SPLITS = 8
 
 def _rows_splits(rows: int, n: int, k: int) -> int:
     """K splits for pc_gemm_rows above GEMM_M128_ROWS rows, or 0 where F.linear (hipBLASLt) is
-    the faster product. By the count of 128 x 128 tiles against the 256 CUs: few tiles want K
-    split (a long K more), and pay for it in partials that the consumer reads; about one per
-    two to four CUs win unsplit; more are the library's. Measured, us of the product alone, here /
-    library: o_proj 7.1 / 9.4 at 256 rows and 9.2 / 11.2 at 512 (2 splits), 13.8 / 15.6 at 1024
-    (unsplit), 22.1 / 22.1 at 2048; down 14.5 / 20.6 at 256, 19.1 / 28.0 at 512, 24.2 / 32.8 at 640
-    (4), 31.3 / 40.0 at 1024 (2), 56.8 / 55.8 at 2048. With weights from HBM and the norm that
-    consumes the output: o_proj at 512 rows 15.5 unsplit, 16.1 at 2 splits; 19.0 / 18.4 at 640; down
-    34.6 / 36.3 at 768 (2)."""
+    the faster product. By the count of 128 x 128 tiles: few of them want K split, a long K more,
+    against partials that the consumer reads; where ours leave CUs idle and the library's do not, it is
+    the library's. Measured inside prefills of the row count, us per layer by which another
+    choice is slower (faster with a minus):
+      o_proj, 2 splits up to 384 rows: library 3.7 at 256 and 2.4 at 288, unsplit 0.4 and 1.1; unsplit to 512:
+      library 1.4, 2 splits 0.0; library to 768: unsplit 0.2 at 576, 0.5 at 768 (-0.2 at 513); unsplit to 1024: library
+      0.9 at 896, 0.9 at 1024 (-0.1 at 769); the library above: unsplit 1.3 at 2048 (-2.3 at 1025);
+      down, 4 splits up to 640 rows: library 5.7 at 256, 6.8 at 640, 2 splits 1.7 and 5.0; 2 splits to 1408: library
+      1.2 at 768, 4.4 at 1024, 3.8 at 1408, 4 splits 9 and more; the library above: 2 splits 26 at 1409 (a
+      second round of tiles), unsplit 6.7."""
     tiles = -(-rows // 128) * -(-n // 128)
     if k >= 4096:
-        return 4 if tiles <= 80 else 2 if tiles <= 128 else 0
-    return 2 if tiles <= 48 else 1 if tiles <= 64 or 100 <= tiles <= 128 else 0
+        return 4 if tiles <= 80 else 2 if tiles <= 176 else 0
+    return 2 if tiles <= 48 else 1 if tiles <= 64 or 112 <= tiles <= 128 else 0
 
 
 def _rows_swiglu(rows: int, width: int) -> bool:
     """Whether pc_gemm_rows runs the SwiGLU projection faster than F.linear + pc_silu_mul: up to
-    one workgroup per CU of 128 x 128 tiles (outputs), or two per CU of 128 x 96, always; beyond
-    that when the last round of 128 x 96 tiles is not mostly empty (1536 rows 77.6 / 84.7 us,
-    2048 rows 95.6 / 101.7; 1280 rows, 590 tiles on 1024 places, 70.6 / 60.1)."""
+    one workgroup per CU of 128 x 128 tiles (outputs), or two per CU of 128 x 96; beyond that when the
+    last round of 128 x 96 tiles is not mostly empty. Us per layer by which the library is
+    slower inside a prefill: 9.1 at 256 rows, 4.4 at 512, 2.6 at 640, 3.0 at 768 (-5 at 769, where this
+    begins its two workgroups per CU; 5.8 at 832), 3.1 at 1024, -20 at 1025, -16 at 1280 (590 tiles on 1024
+    places), -1 at 1408, 1.5 at 1536, 1.1 at 2048."""
     row_tiles = -(-rows // 128)
     if row_tiles * -(-width // 128) <= 256:
         return True
@@ -339,7 +343,7 @@ def _linear_parts(x: Tensor, weight: Tensor, preferred_splits: int) -> Tensor:
 
 def _qkv_fused(rows: int) -> bool:
     """Whether pc_qkv_rope_append is faster than the projection and the RoPE launch after it: up
-    to one 128 x 128 tile per CU (25.5 / 28.6 us at 1536 rows; 33.6 / 33.2 at 2048)."""
+    to one 128 x 128 tile per CU (23.8 / 27.5 us at 1536 rows; 30.4 / 29.7 at 1537, 31.4 / 32.8 at 2048)."""
     return -(-rows // 128) * (QKV_WIDTH // 128) <= 256
 
 

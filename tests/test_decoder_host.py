@@ -265,8 +265,8 @@ def test_rows_splits_always_divide_into_the_decoders_shapes(n, k):
 
 
 def test_rows_whose_k_does_not_divide_are_the_librarys(monkeypatch):
-    """K of one unit cannot be split in two, the count the rule names at this size."""
-    assert dec._rows_splits(129, 128, 64) == 2
+    """65 units of K cannot be split in four, the count the rule names at this size."""
+    assert dec._rows_splits(129, 128, 4160) == 4
     monkeypatch.setattr(_hip, "gemm_rows", lambda *args, **options: pytest.fail("not divisible"))
-    x, weight = torch.ones((129, 64), dtype=torch.float16), torch.ones((128, 64), dtype=torch.float16)
+    x, weight = torch.ones((129, 4160), dtype=torch.float16), torch.ones((128, 4160), dtype=torch.float16)
     assert torch.equal(dec._linear_parts(x, weight, 4), torch.nn.functional.linear(x, weight))

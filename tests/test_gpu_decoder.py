@@ -230,15 +230,15 @@ def test_prefill_paged_matches_the_contiguous_prefill(device, lengths):
         assert torch.equal(after[:, :, others].isnan(), before[:, :, others].isnan())
 
 
-@pytest.mark.parametrize("tokens", [300, 600, 1000])
+@pytest.mark.parametrize("tokens", [200, 300, 600, 1000, 1100])
 def test_long_prefill_with_the_full_mlp_width_is_as_accurate_as_the_reference(device, tokens):
     """Prompts on every route of the projections above 128 rows (o_proj at 2 splits, by the library and
-    unsplit, down at 4 and 2, SwiGLU tiles), with the model's MLP of 5632: logits and the
+    unsplit, down at 4 and 2, SwiGLU tiles and the library's), with the model's MLP of 5632: logits and the
     cached K/V of every layer are as close to the fp32 forward as the reference's own fp16 forward
     is (both evaluated by the oracle's torch expressions on the GPU, attention in fp32)."""
     small = dec.random_weights(device=device, seed=tokens, layers=2, vocab=31, norm_std=0.1)
     weights = dec.TinyLlamaWeights(small.embedding, small.layers * 11, small.final_norm, small.lm_head)
-    allocator = KVAllocator(torch.zeros((22, 2, 64, 16, 4, 64), dtype=torch.float16, device=device))
+    allocator = KVAllocator(torch.zeros((22, 2, 72, 16, 4, 64), dtype=torch.float16, device=device))
     request = RequestId("long")
     allocator.create(KVReservation(request, (tokens + 15) // 16))
     ids = torch.randint(0, 31, (1, tokens), device=device)
