@@ -224,8 +224,11 @@ __device__ __forceinline__ float wave_sum(float x) {
 
 // delta, when given (HAS_DELTA), is fp16 [rows][width] (SPLITS kFp16Input) or fp32 partial sums
 // [splits][rows][width], rounded to fp16 before the add. CHUNKS chunks per thread, all but the last
-// within the row for every thread. All the parameters fit the 64 bytes that are preloaded into SGPRs.
-template <int CHUNKS, bool HAS_DELTA, int SPLITS>
+// within the row for every thread. CLAMP: a thread past the row loads its last chunk again instead of
+// branching round the loads (for rows that fill the workgroup, where it never does: a one-row
+// decode step of 44 norms 784 us, 789 with the branch). All the parameters fit the 64 bytes that are
+// preloaded into SGPRs.
+template <int CHUNKS, bool CLAMP, bool HAS_DELTA, int SPLITS>
 __global__ __launch_bounds__(kNormThreads) void add_rms_norm_kernel(_Float16* hidden, const void* delta,
                                                                     int64_t parts_stride, const _Float16* weight,
                                                                     _Float16* out, int32_t splits, int32_t width,
@@ -238,14 +241,18 @@ __global__ __launch_bounds__(kNormThreads) void add_rms_norm_kernel(_Float16* hi
   const int tid = threadIdx.x;
   half8_t wt[CHUNKS], h[CHUNKS];
   Chunk8<SPLITS> d[CHUNKS];
-  const bool last = tid + (CHUNKS - 1) * kNormThreads < width / 8;
-  auto mine = [&](int k) { return k + 1 < CHUNKS || last; };
-  auto at = [&](int k) { return base + 8 * (tid + k * kNormThreads); };
+  const int chunks = width / 8;
+  auto mine = [&](int k) { return k + 1 < CHUNKS || tid + k * kNormThreads < chunks; };
+  auto column = [&](int k) {
+    const int chunk = tid + k * kNormThreads;
+    return 8 * (CLAMP && chunk >= chunks ? chunks - 1 : chunk);
+  };
+  auto at = [&](int k) { return base + column(k); };
   float squares = 0.0f;
   auto load = [&](int k) {
     if constexpr (HAS_DELTA) d[k] = load8<SPLITS>(delta, at(k), parts_stride);
     h[k] = *reinterpret_cast<const half8_t*>(hidden + at(k));
-    wt[k] = *reinterpret_cast<const half8_t*>(weight + 8 * (tid + k * kNormThreads));
+    wt[k] = *reinterpret_cast<const half8_t*>(weight + column(k));
   };
   auto add = [&](int k) {
     if constexpr (HAS_DELTA) {
@@ -253,28 +260,32 @@ __global__ __launch_bounds__(kNormThreads) void add_rms_norm_kernel(_Float16* hi
 #pragma unroll
       for (int i = 0; i < 8; ++i) h[k][i] = round_h(static_cast<float>(h[k][i]) + static_cast<float>(v[i]));
     }
+    if (!CLAMP || mine(k)) {
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const float x = static_cast<float>(h[k][i]);
-      squares += x * x;
+      for (int i = 0; i < 8; ++i) {
+        const float x = static_cast<float>(h[k][i]);
+        squares += x * x;
+      }
     }
   };
 #pragma unroll
   for (int k = 0; k < CHUNKS; ++k) {
-    if (mine(k)) load(k);
+    if (CLAMP || mine(k)) load(k);
     if constexpr (!kTogether) {
-      if (mine(k)) add(k);
+      if (CLAMP || mine(k)) add(k);
       __builtin_amdgcn_sched_barrier(0);
     }
   }
   if constexpr (kTogether) {
 #pragma unroll
     for (int k = 0; k < CHUNKS; ++k) {
-      if (mine(k)) add(k);
+      if (CLAMP || mine(k)) add(k);
     }
   }
   squares = wave_sum(squares);
   if ((tid & 63) == 0) wave_sums[tid >> 6] = squares;
+  // The barrier also orders every thread's residual loads before the first store (CLAMP: a chunk may be
+  // loaded by more threads than the one that stores it).
   __syncthreads();
   float total = 0.0f;
 #pragma unroll
@@ -374,10 +385,11 @@ int add_rms_norm(void* out, void* hidden, const void* delta, const float* delta_
     constexpr int S = decltype(instance)::value;
     static_assert(kNormMaxChunks == 4, "one instance per chunk count");
     switch ((width / 8 - 1) / kNormThreads) {
-      case 0: return launch(add_rms_norm_kernel<1, D, S>);
-      case 1: return launch(add_rms_norm_kernel<2, D, S>);
-      case 2: return launch(add_rms_norm_kernel<3, D, S>);
-      default: return launch(add_rms_norm_kernel<4, D, S>);
+      case 0:
+        return width == 8 * kNormThreads ? launch(add_rms_norm_kernel<1, true, D, S>) : launch(add_rms_norm_kernel<1, false, D, S>);
+      case 1: return launch(add_rms_norm_kernel<2, false, D, S>);
+      case 2: return launch(add_rms_norm_kernel<3, false, D, S>);
+      default: return launch(add_rms_norm_kernel<4, false, D, S>);
     }
   };
   if (delta == nullptr && delta_parts == nullptr) {
