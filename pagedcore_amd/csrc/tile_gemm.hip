@@ -302,8 +302,8 @@ namespace gemm_device {
 // RoPE epilogue: the smallest tile of which every CU gets at most one, as above, with a stage
 // more where it fits (us, against this file's partials or hipBLASLt and pc_rope_kv_append: 64 x 64
 // at 384 rows 12.5 / 14.5, three stages 14.5; 128 x 64 at 512 rows 17.0 / 18.0, at 768 17.4 / 20.3;
-// 128 x 128 at 1024 rows 25.1 / 26.5, at 1536 25.5 / 28.6). Larger than that it ties: 33.6 / 33.2 at
-// 2048 rows.
+// 128 x 128 at 1024 rows 25.1 / 26.5, at 1536 25.5 / 28.6). Larger than that it ties (33.6 / 33.2 at
+// 2048 rows), and the decoder leaves it to hipBLASLt: 128 x 192 serves direct calls.
 int launch_qkv_rows(const QkvArgs& q, hipStream_t s) {
   const TileArgs a{q.x, q.w, q.m, kQkvElems, q.k, q.k, nullptr};
   if (tile_count(a, 64, 64, a.n) <= kCUs) return launch<64, 64, 2, 2, 4, kRope>(a, q.positions, q.slots, q.out, s);
