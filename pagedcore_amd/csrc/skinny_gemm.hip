@@ -40,6 +40,7 @@ using pc_internal::set_error;
 
 constexpr int kMaxRows = 128;
 constexpr int kMaxQkvK = 1 << 18;  // 2560 rows of W within 32-bit offsets
+constexpr int kMaxStreamK = 1 << 24;  // gemm_stream_kernel: 64 rows within 32-bit offsets
 constexpr int kSwiGLUHalf = 32;  // gate (and up) rows per SwiGLU tile
 
 struct GemmArgs {
@@ -588,7 +589,7 @@ namespace gemm_device {
 // order; k from 256, where every wave has a unit). It and narrower products are also faster here than on 64 x 64 tiles (us: n 2560 at 160
 // rows 6.9 / 10.5, at 288 9.5 / 10.6; n 2048 at 256 rows 7.0 / 10.4; n 512 4.9 / 10.3), wider ones
 // hardly or not (n 5632 at 160 rows 14.6 / 14.9, at 96 12.2 / 11.5).
-bool rows_stream(int m, int n, int k) { return m <= kMaxStreamQkv && n <= kQkvElems && k >= 256; }
+bool rows_stream(int m, int n, int k) { return m <= kMaxStreamQkv && n <= kQkvElems && k >= 256 && k <= kMaxStreamK; }
 
 int launch_rows_stream(void* out, const _Float16* x, const _Float16* w, int m, int n, int k, Epilogue epilogue,
                        hipStream_t s) {
@@ -614,7 +615,7 @@ namespace {
 // the same kernel (each projection of the decoder from 1 to 64 rows, and from 65 to 128).
 constexpr float kMargin = 1.1f;  // where the estimates are close, gemm_m128_kernel
 bool stream_form(const GemmArgs& a, int splits) {
-  if (a.ksplit % 64 != 0 || a.k > (1 << 24)) return false;  // row offsets in 32 bits
+  if (a.ksplit % 64 != 0 || a.k > kMaxStreamK) return false;
   if (splits == 1 && rows_stream(a.m, a.n, a.k)) return true;
   // A K range of fewer units than waves leaves waves idle (n 1024, k 128 per split, 48 rows: 3.5
   // us / 3.1; k 64, n 15488, SwiGLU at 12 rows 4.2 / 3.2).

@@ -296,6 +296,25 @@ def test_gemm_forms(device, m, n, k, splits):
             assert np.array_equal(_bits(fused[: m * (n // 2)]), _bits(separate.view(-1)))
 
 
+@pytest.mark.parametrize("epilogue", [_hip.GEMM_PARTIALS, _hip.GEMM_HALF])
+def test_gemm_of_the_longest_k(device, epilogue):
+    """K past the streams' 32-bit row offsets (2^24), few columns: small integers in a few columns of K
+    at both ends and across the limit, so that every sum is exact."""
+    m, n, k = 17, 32, (1 << 24) + 64
+    columns = torch.tensor([0, 63, 64, (1 << 23) + 5, (1 << 24) - 1, 1 << 24, (1 << 24) + 1, k - 1], device=device)
+    gen = torch.Generator(device=device).manual_seed(1)
+    few_x = torch.randint(-4, 5, (m, len(columns)), device=device, generator=gen).half()
+    few_w = torch.randint(-4, 5, (n, len(columns)), device=device, generator=gen).half()
+    x, w = (torch.zeros((rows, k), dtype=torch.float16, device=device) for rows in (m, n))
+    x[:, columns], w[:, columns] = few_x, few_w
+    expected = few_x.double() @ few_w.double().T
+    out = torch.full((1, m, n) if epilogue == _hip.GEMM_PARTIALS else (m, n), float("nan"), device=device,
+                     dtype=torch.float32 if epilogue == _hip.GEMM_PARTIALS else torch.float16)
+    _hip.gemm_m128(out, x, w, epilogue=epilogue)
+    torch.cuda.synchronize()
+    assert torch.equal(out.view(m, n).double(), expected)
+
+
 @pytest.mark.parametrize("rows,full", [(1, 64), (16, 64), (17, 64), (33, 64), (48, 64), (49, 64), (65, 128), (80, 128), (81, 128), (97, 128)])
 def test_decoder_projections_do_not_depend_on_the_batch(device, rows, full):
     """The projections a decode step issues, at its split counts: a row has the same bits in every batch
