@@ -252,6 +252,8 @@ def _check_weights(weights: TinyLlamaWeights, what: str) -> None:
 # Up to 64 rows half as many for o_proj and down: the kernel that runs there fills the GPU
 # with them (o_proj 3.4-4.1 us at 2 splits, 3.4-4.4 at 4; down 5.9-8.5 at 4, 6.0-7.8 at 8) and
 # the norm that sums the partials reads half.
+# So a row has the same bits in every batch of up to 64 rows, and in every batch of 65 to 128, but
+# not in one of each: the sums are in another order.
 GEMM_M128_ROWS = 128
 GEMM_FEW_ROWS = 64
 QKV_SPLITS = 1
@@ -382,10 +384,10 @@ def _swiglu(x: Tensor, gate_up: Tensor) -> Tensor:
     rows, k = x.shape
     n = gate_up.shape[0]
     activated = torch.empty((rows, n // 2), dtype=torch.float16, device=x.device)
-    fits = n % 64 == 0 and k % 64 == 0 and _rows_fit(rows, n, k) and _kernel_operands(x, gate_up)
+    fits = n % 64 == 0 and k % 64 == 0 and _kernel_operands(x, gate_up)
     if fits and rows <= GEMM_M128_ROWS:
         _hip.gemm_m128(activated, x, gate_up, epilogue=_hip.GEMM_SWIGLU)
-    elif fits and _rows_swiglu(rows, n // 2):
+    elif fits and _rows_fit(rows, n, k) and _rows_swiglu(rows, n // 2):
         _hip.gemm_rows(activated, x, gate_up, epilogue=_hip.GEMM_SWIGLU)
     else:
         _hip.silu_mul(activated, F.linear(x, gate_up))
