@@ -526,11 +526,11 @@ M128Tile m128_tile(int n, int splits) {
 // rounds of workgroups on the CUs times a round's setup and the bytes it moves into a CU. A later
 // round overlaps an earlier one where workgroups share a CU (two of up to 80 KB of LDS; three of 48 KB,
 // while a K range is short enough for the L2 to hold what they share). The constants are fitted to
-// the times of every form at 22800 calls (m 1 to 128, n 32 to 37000, k 64 to 16000, 1 to 16
+// the times of every form at 23000 calls (m 1 to 128, n 32 to 37000, k 64 to 16000, 1 to 16
 // splits, weights from HBM): the form taken is 2 % off the fastest on average; it is more than 5 %
-// slower than gemm_m128_kernel alone at 0.4 % of them (17 % at most) and 36 % faster on average. A
-// rule on the number of W tiles was more than 5 % slower at 11 % of them, by up to 56 % (SwiGLU of n 14336
-// at 64 rows 20.7 / 15.0, 299 tiles of 48 rows; n 7136, k 256 at 111 rows 5.8 / 4.1).
+// slower than gemm_m128_kernel alone at 0.4 % of them (17 % at most) and 35 % faster on average. A
+// rule on the number of W tiles was more than 5 % slower at 15 % of them, by up to 2.2 times (SwiGLU of n
+// 14336 at 64 rows 20.7 / 15.0, 299 tiles of 48 rows; n 7136, k 256 at 111 rows 5.8 / 4.1).
 float stream_time(const GemmArgs& a, int splits, StreamTile t) {
   const int64_t workgroups =
       static_cast<int64_t>((a.n + 16 * t.nt - 1) / (16 * t.nt)) * splits * ((a.m + 16 * t.mt - 1) / (16 * t.mt));
